@@ -56,6 +56,8 @@ def kernel_bytes(cfg, mixed):
         "k_cn": nf * Cj_t + (nf + 1) * C + (2.0 / 3.0) * nf * Cj + nf * Cj + nf * C,
         "k_project": 4 * C + 4 * C,
     }
+    # DNS: the same with the projection in the kernel: the pressure goes out too
+    out["k_column"] = out["k_cn"] + C
     if cfg.use_les:
         # physical fields: R8 FP64, Rt in the transform precision; na SGS addition fields
         R8 = cfg.nx * cfg.nz * 8 * ny2

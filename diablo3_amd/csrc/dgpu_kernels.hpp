@@ -262,23 +262,22 @@ __global__ __launch_bounds__(NT) void k_fwd_x(Ptrs<const T*, MAXO> src, Ptrs<cx<
 // (the reference evaluates them inline; the host table holds the same quotients).
 enum RowCoef {
   RC_RDY = 0,    // 1/dy(j)
-  RC_RDYP,       // 1/dy(j+1)
   RC_RDYF,       // 1/dyf(j)
-  RC_RDYFM,      // 1/dyf(j-1)
   RC_WTH,        // dyf(j-1)/(2 dy(j)): weight of th(j) in the GY interpolation
   RC_WTHM,       // dyf(j)/(2 dy(j)):   weight of th(j-1)
   RC_FLO,        // 1/(dy(j) dyf(j)):    lower coupling of a GYF row (u1, u3, scalars)
   RC_FHI,        // 1/(dy(j+1) dyf(j)):  upper coupling of a GYF row
   RC_GLO,        // 1/(dyf(j-1) dy(j)):  lower coupling of a GY row (u2)
   RC_GHI,        // 1/(dyf(j) dy(j)):    upper coupling of a GY row
+  RC_TW0,        // per scalar n, 4 entries at RC_TW0 + 4n:
+  // +0 dthdx (gyf-Ly/2) delta/Ro_inv, +1 -dthdz (gyf-Ly/2) delta/Ro_inv,
+  // +2 dthdx (gy-Ly/2) delta/Ro_inv,  +3 -dthdz (gy-Ly/2) delta/Ro_inv
+  RC_RDYFM = RC_TW0 + 4 * MAXTH,  // 1/dyf(j-1)
   RC_YX,         // 2 dy(j) / (dx beta_sgs):  the AMD closure's width ratios at GY j
   RC_XY,         // (dx beta_sgs) / (2 dy(j))
   RC_YZ,         // 2 dy(j) / (dz beta_sgs)
   RC_ZY,         // (dz beta_sgs) / (2 dy(j))
-  RC_TW0,        // per scalar n, 4 entries at RC_TW0 + 4n:
-  RC_COUNT = RC_TW0 + 4 * MAXTH
-  // +0 dthdx (gyf-Ly/2) delta/Ro_inv, +1 -dthdz (gyf-Ly/2) delta/Ro_inv,
-  // +2 dthdx (gy-Ly/2) delta/Ro_inv,  +3 -dthdz (gy-Ly/2) delta/Ro_inv
+  RC_COUNT
 };
 
 struct XProdArgs {
@@ -710,32 +709,8 @@ __global__ __launch_bounds__(NT) void k_fwdz_nl(NlArgs a, int ntiles) {
 }
 
 // ---------------------------------------------------------------------------
-// filter_chan (for/solver.f90:1597-1685): the horizontal filter of one scalar,
-// cth *= sigma(kx, kz) on rows [jlo, jhi]; sigma [kzr][kxp] from the host
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_filter_th(Geo g, cd* __restrict__ th, const double* __restrict__ sigma,
-                                                     int jlo, int jhi) {
-  const long long c = (long long)blockIdx.x * 256 + threadIdx.x;
-  const int j = jlo + blockIdx.y;
-  if (c >= g.pc || j > jhi) return;
-  if (c % g.kxp >= g.kxr) return;
-  const long long o = (long long)j * g.pc + c;
-  th[o] = sigma[c] * th[o];
-}
-
-// ---------------------------------------------------------------------------
-// Column kernel.  Per (kx, kz) column and all rows j = 0..Nyp+1:
-//  1. Fourier-space assembly of rk_chan_1 (for/solver.f90:385-838, 909-973, and
-//     user_rhs_chan_fourier 35-111): new RK memory cf and the right-hand side cr,
-//     including the explicit half of Crank–Nicolson (for/solver.f90:850-870,
-//     981-1002) and the BC rows of apply_BC_* (for/solver.f90:1901-2232);
-//  2. the Crank–Nicolson solves of every scalar, then u2, u1, u3
-//     (for/solver.f90:1004-1233), in Fourier space (the DNS operator does not
-//     depend on x or z), by parallel cyclic reduction with coefficients that the
-//     host precomputes from the reference's matrices;
-//  3. rem_div_chan (for/solver.f90:1302-1379, BC rows 2330-2371) by parallel cyclic
-//     reduction, then the velocity correction and the pressure update
-//     (for/solver.f90:1261-1267).
+// Arguments and the Fourier-space assembly of the column kernels (dgpu_column.hpp)
+// and of k_assemble.
 // ---------------------------------------------------------------------------
 
 struct SolveRows {
@@ -747,30 +722,31 @@ struct SolveRows {
 
 struct ColArgs {
   Geo g;
-  int rk, do_cn, plevels;
-  int cr_minus_u;   // do_cn == 0: write the right-hand side minus the state (increment solves)
+  int rk;
+  int cr_minus_u;   // k_assemble: write the right-hand side minus the state (increment solves)
   int jstart, jend, jstart_th[MAXTH], jend_th[MAXTH];
   int front, f_type;
   double nu, beta, nu_v_scale, ro_inv, delta, grav_x, grav_y, grav_z, ly, px0, omega0, amp_omega0, time;
   double pr[MAXTH], dthdx[MAXTH], dthdz[MAXTH];
   double temp1, temp3, temp4, temp5;
-  // host-precomputed scalars: Ro_inv/delta; per scalar dthdx delta/Ro_inv,
-  // -dthdz delta/Ro_inv, nu/Pr, temp1 nu_v_scale/Pr; temp1 nu_v_scale
-  double cori, twu_x[MAXTH], twu_z[MAXTH], nupr[MAXTH], t1pr[MAXTH], t1v;
+  // host-precomputed scalars: Ro_inv/delta; the scalars' sums of dthdx delta/Ro_inv
+  // and -dthdz delta/Ro_inv (0 without the thermal wind); per scalar nu/Pr,
+  // temp1 nu_v_scale/Pr; temp1 nu_v_scale
+  double cori, twu_x, twu_z, nupr[MAXTH], t1pr[MAXTH], t1v;
+  double twon;   // 1 with the front's thermal-wind terms, else 0
   const double* __restrict__ rowc;  // [ny2][RC_COUNT]
   const double *__restrict__ dy, *__restrict__ dyf, *__restrict__ gy, *__restrict__ gyf;
   const double *__restrict__ kx, *__restrict__ kz;
   SolveRows rows[MAXF];
-  // Thomas factorisation of the CN systems, [field][ny2][5]: mu_j (forward
-  // multiplier), beta_j = 1/b'_j, gamma_j = -c_j/b'_j, F_j / G_j (products of mu /
-  // gamma from the chunk start / to the chunk end); rows per chunk
+  unsigned long long bcmask;  // bit MAXF s + e: row s of SolveRows::kind is a BC row of field e
+  // Thomas factorisation of the CN systems, [field][3][ny2]: mu_j (forward
+  // multiplier), beta_j = 1/b'_j, gamma_j = -c_j/b'_j
   const double* __restrict__ thc;
-  int chunk;
   cd* u[MAXF];
   cd* p;
   cd* cf[MAXF];
   const void* nl[MAXF];
-  cd* crout[MAXF];  // do_cn == 0: right-hand side rows [blo, bhi] of the physical-space solve
+  cd* crout[MAXF];  // k_assemble: right-hand side rows [blo, bhi] of the physical-space solve
   // k_project in its poisson_p_chan form: the transformed source (else null), the
   // scalar count for its buoyancy term; the solution goes to p
   const cd* prhs;
@@ -787,107 +763,81 @@ __device__ __forceinline__ int xcd_tile(int b, int nb) {
   return t < nb ? t : -1;
 }
 
-__device__ __forceinline__ int special_row(int j, int ny) {
-  return j <= 2 ? j : (j == ny ? 3 : (j == ny + 1 ? 4 : -1));
-}
-
-// Inputs of the assembly at one (row j, column) point.  Loaded before any store
-// so that the loads of a thread's rows are independent of its cf stores.
+// Inputs of the assembly at one (row j, column) point, fields u1, u2, u3, th_n:
+// the state on rows j-1, j, j+1, the pressure on j-1, j, the old RK memory and
+// the nonlinear terms.
 template <int NTH>
 struct RowIn {
-  cd u1m, u1c, u1p, u2m, u2c, u2p, u3m, u3c, u3p, pm, pc_;
-  cd thm[NTH > 0 ? NTH : 1], thc[NTH > 0 ? NTH : 1], thp[NTH > 0 ? NTH : 1];
-  cd cfo[3 + NTH], nl[3 + NTH];
+  cd um[3 + NTH], uc[3 + NTH], up[3 + NTH], pm, pc_, cfo[3 + NTH], nl[3 + NTH];
 };
 
-template <typename T, int NTH>
-__device__ __forceinline__ void load_row(RowIn<NTH>& r, const ColArgs& a, long long o, long long pc,
-                                         const cd* __restrict__ u1, const cd* __restrict__ u2,
-                                         const cd* __restrict__ u3, const cd* __restrict__ t0,
-                                         const cd* __restrict__ t1, const cd* __restrict__ p) {
-  const long long om = o - pc, op = o + pc;
-  r.u1m = u1[om]; r.u1c = u1[o]; r.u1p = u1[op];
-  r.u2m = u2[om]; r.u2c = u2[o]; r.u2p = u2[op];
-  r.u3m = u3[om]; r.u3c = u3[o]; r.u3p = u3[op];
-  r.pm = p[om]; r.pc_ = p[o];
-  if constexpr (NTH >= 1) { r.thm[0] = t0[om]; r.thc[0] = t0[o]; r.thp[0] = t0[op]; }
-  if constexpr (NTH >= 2) { r.thm[1] = t1[om]; r.thc[1] = t1[o]; r.thp[1] = t1[op]; }
+// Per-column constants of the assembly: the wavenumbers, (kx^2 + kz^2)^beta, and
+// the wavenumbers that the thermal wind's advection takes (0 without it).
+struct ColK {
+  double kx, kz, kk, kxt, kzt, gyb;
+};
+__device__ __forceinline__ ColK col_k(const ColArgs& a, double kx, double kz, bool mean) {
+  const double k2 = kx * kx + kz * kz;
+  return {kx, kz, (a.beta == 1.0) ? k2 : pow(k2, a.beta), a.twon * kx, a.twon * kz, mean ? 0.0 : a.grav_y};
+}
+
+// cf and cr of every equation at one point (for/solver.f90:385-838, 850-870,
+// 981-1002 and user_rhs_chan_fourier 35-111); rc[RowCoef] the row's coefficients.
+// The linear terms of one field share a form: -damp u - i s u, with the thermal
+// wind's advection in s.
+template <int NTH, typename RC>
+__device__ __forceinline__ void assemble_row(const ColArgs& a, const RowIn<NTH>& r, const RC rc, const ColK& K, cd* cf,
+                                             cd* cr) {
+  double sf[NTH > 0 ? NTH : 1], sft = 0.0, sgt = 0.0;
+#pragma unroll
+  for (int n = 0; n < NTH; ++n) {
+    sf[n] = rc[RC_TW0 + 4 * n] * K.kzt + rc[RC_TW0 + 4 * n + 1] * K.kxt;
+    sft = sft + sf[n];
+    sgt = sgt + (rc[RC_TW0 + 4 * n + 2] * K.kzt + rc[RC_TW0 + 4 * n + 3] * K.kxt);
+  }
+  const double damp = a.nu * K.kk;
+  auto lin = [](cd u, double d, double s) { return cd{s * u.y - d * u.x, -(s * u.x) - d * u.y}; };
+  // u1 and u3
+  const cd u2m = 0.5 * (r.uc[1] + r.up[1]);
+  cf[0] = lin(r.uc[0], damp, sft) + a.cori * r.uc[2] - a.twu_z * u2m + r.nl[0];
+  cf[2] = lin(r.uc[2], damp, sft) - a.cori * r.uc[0] - a.twu_x * u2m + r.nl[2];
+  // u2 (the buoyancy not in the mean mode)
+  cf[1] = lin(r.uc[1], damp, sgt) + r.nl[1];
+#pragma unroll
+  for (int n = 0; n < NTH; ++n) {
+    const cd t = r.uc[3 + n];
+    cf[0] = cf[0] + a.grav_x * t;
+    cf[2] = cf[2] + a.grav_z * t;
+    cf[1] = cf[1] + (K.gyb * rc[RC_WTH]) * t + (K.gyb * rc[RC_WTHM]) * r.um[3 + n];
+    cf[3 + n] = lin(t, a.nupr[n] * K.kk, sf[n]) - a.dthdx[n] * r.uc[0] - a.dthdz[n] * r.uc[2] + r.nl[3 + n];
+  }
+  const double flo = rc[RC_FLO], fhi = rc[RC_FHI];
+  const double px = a.temp4 * K.kx, pz = a.temp4 * K.kz;
 #pragma unroll
   for (int e = 0; e < 3 + NTH; ++e) {
-    r.cfo[e] = (a.rk > 1) ? ((const cd* __restrict__)a.cf[e])[o] : cd{0.0, 0.0};
-    r.nl[e] = cvt<double>(((const cx<T>* __restrict__)a.nl[e])[o]);
+    const double t1 = e < 3 ? a.t1v : a.t1pr[e < 3 ? 0 : e - 3];
+    const double lo = t1 * (e == 1 ? rc[RC_GLO] : flo), hi = t1 * (e == 1 ? rc[RC_GHI] : fhi);
+    cd v = r.uc[e] + a.temp3 * r.cfo[e];
+    if (e == 0) v = v - ik(px, r.pc_);
+    if (e == 1) v = v - (a.temp4 * rc[RC_RDY]) * (r.pc_ - r.pm);
+    if (e == 2) v = v - ik(pz, r.pc_);
+    v = v + a.temp5 * cf[e];
+    cr[e] = v + hi * (r.up[e] - r.uc[e]) - lo * (r.uc[e] - r.um[e]);
   }
 }
 
-// cf and cr of equation e at row j, column (i, k), from the loaded row inputs;
-// kk = (kx^2 + kz^2)^beta of the column, rc the row's coefficient table
-template <int NTH>
-__device__ __forceinline__ void assemble(const ColArgs& a, const RowIn<NTH>& r, const double* __restrict__ rc,
-                                         int e, int i, int k, double kxi, double kzk, double kk,
-                                         cd& cf, cd& cr) {
-  const bool tws = a.front && a.ro_inv != 0.0;
-  if (e == 0 || e == 2) {
-    const cd uc = (e == 0) ? r.u1c : r.u3c;
-    const cd up = (e == 0) ? r.u1p : r.u3p;
-    const cd um = (e == 0) ? r.u1m : r.u3m;
-    cf = -1.0 * ((a.nu * kk) * uc);
-    if (e == 0) cf = cf + a.cori * r.u3c;
-    else cf = cf - a.cori * r.u1c;
-    for (int n = 0; n < NTH; ++n) cf = cf + (e == 0 ? a.grav_x : a.grav_z) * r.thc[n];
-    if (tws) {
-      const cd u2m = 0.5 * (r.u2c + r.u2p);
-      for (int n = 0; n < NTH; ++n) {
-        cf = cf - rc[RC_TW0 + 4 * n] * ik(kzk, uc) - rc[RC_TW0 + 4 * n + 1] * ik(kxi, uc);
-        if (e == 0) cf = cf - a.twu_z[n] * u2m;
-        else cf = cf - a.twu_x[n] * u2m;
-      }
-    }
-    cf = cf + r.nl[e];
-    cr = uc;
-    if (a.rk > 1) cr = cr + a.temp3 * r.cfo[e];
-    cr = cr - a.temp4 * (e == 0 ? ik(kxi, r.pc_) : ik(kzk, r.pc_));
-    if (e == 0 && k == 0 && i == 0) {
-      if (a.f_type == 1) cr.x = cr.x - a.temp4 * a.px0;
-      else if (a.f_type == 2) cr.x = cr.x - a.temp4 * (a.px0 + a.amp_omega0 * cos(a.omega0 * a.time));
-    }
-    cr = cr + a.temp5 * cf;
-    cr = cr + a.t1v * (rc[RC_RDYF] * (rc[RC_RDYP] * (up - uc) - rc[RC_RDY] * (uc - um)));
-  } else if (e == 1) {
-    const cd uc = r.u2c;
-    cf = -1.0 * ((a.nu * kk) * uc);
-    if (!(k == 0 && i == 0)) {
-      for (int n = 0; n < NTH; ++n) cf = cf + a.grav_y * (rc[RC_WTH] * r.thc[n] + rc[RC_WTHM] * r.thm[n]);
-    }
-    if (tws) {
-      for (int n = 0; n < NTH; ++n)
-        cf = cf - rc[RC_TW0 + 4 * n + 2] * ik(kzk, uc) - rc[RC_TW0 + 4 * n + 3] * ik(kxi, uc);
-    }
-    cf = cf + r.nl[1];
-    cr = uc;
-    if (a.rk > 1) cr = cr + a.temp3 * r.cfo[1];
-    cr = cr - a.temp4 * (rc[RC_RDY] * (r.pc_ - r.pm));
-    cr = cr + a.temp5 * cf;
-    cr = cr + a.t1v * (rc[RC_RDY] * (rc[RC_RDYF] * (r.u2p - uc) - rc[RC_RDYFM] * (uc - r.u2m)));
-  } else {
-    const int n = e - 3;
-    const cd tc = r.thc[n];
-    cf = -1.0 * ((a.nupr[n] * kk) * tc);
-    cf = cf - a.dthdx[n] * r.u1c - a.dthdz[n] * r.u3c;
-    if (tws) cf = cf - rc[RC_TW0 + 4 * n] * ik(kzk, tc) - rc[RC_TW0 + 4 * n + 1] * ik(kxi, tc);
-    cf = cf + r.nl[e];
-    cr = tc;
-    if (a.rk > 1) cr = cr + a.temp3 * r.cfo[e];
-    cr = cr + a.temp5 * cf;
-    cr = cr + a.t1pr[n] * (rc[RC_RDYF] * (rc[RC_RDYP] * (r.thp[n] - tc) - rc[RC_RDY] * (tc - r.thm[n])));
-  }
+// The mean pressure gradient of f_type 1 and 2 in u1's (0, 0) mode.
+__device__ __forceinline__ double mean_dpdx(const ColArgs& a) {
+  if (a.f_type == 1) return a.temp4 * a.px0;
+  if (a.f_type == 2) return a.temp4 * (a.px0 + a.amp_omega0 * cos(a.omega0 * a.time));
+  return 0.0;
 }
 
-// The assembly of k_cn alone (the LES branch, whose CN solve runs per physical
+// The assembly of k_column alone (the LES branch, whose CN solve runs per physical
 // column): cf and the right-hand side (or the right-hand side minus the state,
 // cr_minus_u) of every equation at one point per thread.  The columns of a row
 // are consecutive threads, so every load and store of a wave is one contiguous
-// run of the plane, and no LDS is held (the column kernel reserves its solve's).
-// Same rows, same load_row / assemble, same writes as k_cn with do_cn = 0.
+// run of the plane.
 template <typename T, int NTH>
 __global__ __launch_bounds__(256) void k_assemble(ColArgs a) {
   constexpr int NF = 3 + NTH;
@@ -896,339 +846,38 @@ __global__ __launch_bounds__(256) void k_assemble(ColArgs a) {
   const int j = blockIdx.y;
   if (c >= g.pc) return;
   const int i = (int)(c % g.kxp), k = (int)(c / g.kxp);
-  if (i >= g.kxr) return;  // padding columns: k_cn writes nothing there either
+  if (i >= g.kxr) return;  // padding columns: k_column writes nothing there either
   const long long pc = g.pc;
-  const double kxi = a.kx[i], kzk = a.kz[k];
-  const double k2 = kxi * kxi + kzk * kzk;
-  const double kk = (a.beta == 1.0) ? k2 : pow(k2, a.beta);
+  const ColK K = col_k(a, a.kx[i], a.kz[k], c == 0);
   const long long o = (long long)j * pc + c;
   const bool inner = j >= 1 && j <= g.ny;
   RowIn<NTH> r;
-  if (inner)
-    load_row<T, NTH>(r, a, o, pc, a.u[0], a.u[1], a.u[2], NTH >= 1 ? a.u[3] : a.u[0], NTH >= 2 ? a.u[4] : a.u[0],
-                     a.p);
+  cd cf[NF], cr[NF];
+  if (inner) {
+#pragma unroll
+    for (int e = 0; e < NF; ++e) {
+      const cd* __restrict__ u = a.u[e];
+      r.um[e] = u[o - pc]; r.uc[e] = u[o]; r.up[e] = u[o + pc];
+    }
+    r.pm = a.p[o - pc]; r.pc_ = a.p[o];
+#pragma unroll
+    for (int e = 0; e < NF; ++e) {
+      r.cfo[e] = (a.rk > 1) ? ((const cd* __restrict__)a.cf[e])[o] : cd{0.0, 0.0};
+      r.nl[e] = cvt<double>(((const cx<T>* __restrict__)a.nl[e])[o]);
+    }
+    assemble_row<NTH>(a, r, a.rowc + (long long)j * RC_COUNT, K, cf, cr);
+    if (c == 0) cr[0].x = cr[0].x - mean_dpdx(a);
+  }
 #pragma unroll
   for (int e = 0; e < NF; ++e) {
     const SolveRows& SR = a.rows[e];
     cd v = {0.0, 0.0};
     if (inner && j >= SR.blo && j <= SR.bhi) {
-      cd cf;
-      assemble<NTH>(a, r, a.rowc + (long long)j * RC_COUNT, e, i, k, kxi, kzk, kk, cf, v);
-      a.cf[e][o] = cf;
-      if (a.cr_minus_u) v = v - a.u[e][o];
+      v = cr[e];
+      a.cf[e][o] = cf[e];
+      if (a.cr_minus_u) v = v - r.uc[e];
     }
     a.crout[e][o] = v;
-  }
-}
-
-// Assembly + Crank-Nicolson solves.  T: precision of the nonlinear terms;
-// TC columns x RG row groups per block; RPT >= ceil(ny2 / RG) rows per thread.
-// The CN solution overwrites the state rows [wlo, whi]; k_project follows.
-template <typename T, int TC, int NT, int RPT, int NTH, int LMAX>
-__global__ __launch_bounds__(NT) void k_cn(ColArgs a) {
-  constexpr int NF = 3 + NTH;
-  constexpr int RG = NT / TC;
-  extern __shared__ unsigned char smem[];
-  const Geo& g = a.g;
-  const int ny2 = g.ny2, ny = g.ny, tid = threadIdx.x;
-  const int cc = tid % TC, rg = tid / TC;
-  const int tile = xcd_tile(blockIdx.x, (int)(g.pc / TC));
-  if (tile < 0) return;
-  const int c = tile * TC + cc;  // column in the padded plane: c = k*kxp + i
-  const int i = c % g.kxp, k = c / g.kxp;
-  const bool active = i < g.kxr;
-  const long long pc = g.pc;
-  cd* sR = (cd*)smem;
-  // rows of the TC columns interleaved: lanes of one row group touch consecutive 16-byte slots
-  auto R = [&](int f, int j) -> cd& { return sR[(f * ny2 + j) * TC + cc]; };
-  const cd* __restrict__ u1 = a.u[0];
-  const cd* __restrict__ u2 = a.u[1];
-  const cd* __restrict__ u3 = a.u[2];
-  const cd* __restrict__ t0 = NTH >= 1 ? a.u[3] : a.u[0];
-  const cd* __restrict__ t1 = NTH >= 2 ? a.u[4] : a.u[0];
-  const cd* __restrict__ pp = a.p;
-
-  // ---- 1. assembly of cf and cr; BC rows of the right-hand side
-  const double kxi = active ? a.kx[i] : 0.0, kzk = a.kz[k];
-  const double k2 = kxi * kxi + kzk * kzk;
-  const double kk = (a.beta == 1.0) ? k2 : pow(k2, a.beta);
-  for (int m = 0; m < RPT; ++m) {
-    const int j = rg + m * RG;
-    if (j >= ny2) break;
-    const long long o = (long long)j * pc + c;
-    const bool inner = active && j >= 1 && j <= ny;
-    RowIn<NTH> r;
-    if (inner) load_row<T, NTH>(r, a, o, pc, u1, u2, u3, t0, t1, pp);
-    cd crv[NF];
-#pragma unroll
-    for (int e = 0; e < NF; ++e) {
-      const SolveRows& SR = a.rows[e];
-      cd v = {0.0, 0.0};
-      if (inner && j >= SR.blo && j <= SR.bhi) {
-        cd cf;
-        assemble<NTH>(a, r, a.rowc + (long long)j * RC_COUNT, e, i, k, kxi, kzk, kk, cf, v);
-        a.cf[e][o] = cf;
-      }
-      if (a.do_cn) {
-        const int sr = special_row(j, ny);
-        const int kd = sr >= 0 ? SR.kind[sr] : -1;
-        if (kd == 0) v = {0.0, 0.0};
-        else if (kd == 1) v = (c == 0) ? cd{SR.val[sr], 0.0} : cd{0.0, 0.0};
-        else if (!(j >= SR.blo && j <= SR.bhi)) v = {0.0, 0.0};
-      } else if (!(inner && j >= SR.blo && j <= SR.bhi)) {
-        v = {0.0, 0.0};  // physical-space solve: its BC rows are set per column there
-      }
-      crv[e] = v;
-    }
-    if (!a.do_cn) {
-      if (active) {
-#pragma unroll
-        for (int e = 0; e < NF; ++e) {
-          cd v = crv[e];
-          if (a.cr_minus_u && inner && j >= a.rows[e].blo && j <= a.rows[e].bhi) v = v - a.u[e][o];
-          a.crout[e][o] = v;
-        }
-      }
-      continue;
-    }
-#pragma unroll
-    for (int e = 0; e < NF; ++e) R(e, j) = crv[e];
-  }
-  if (!a.do_cn) return;  // uniform over the grid
-  __syncthreads();
-
-  // ---- 2. Thomas with the host's factorisation, in chunks.  One wave takes one
-  // field of the TC columns: lane = p*TC + cc, p = chunk of L consecutive rows.
-  // Per chunk: local elimination from zero, a shuffle scan of the chunk-boundary
-  // carries (the affine maps y -> A y + B compose), and the fix-up with the
-  // host's in-chunk products.  Same linear map as thomas_forward/backward_real_mpi
-  // (for/solver.f90:1691-1761, 1816-1852); scalars first (for/solver.f90:1004-1007).
-  constexpr int P = 64 / TC;
-  const int lane = tid & 63, wave = tid / 64;
-  const int p = lane / TC, ccl = lane % TC;
-  const int L = a.chunk, j0 = p * L;
-  const int cl = tile * TC + ccl;
-  const bool act_l = (cl % g.kxp) < g.kxr;
-  for (int e0 = wave; e0 < NF; e0 += NT / 64) {
-    const int e = (e0 < NTH) ? 3 + e0 : e0 - NTH;
-    const double* __restrict__ co = a.thc + (long long)e * ny2 * 5;  // mu, beta, gamma, F, G per row
-    auto Rl = [&](int j) -> cd& { return sR[(e * ny2 + j) * TC + ccl]; };
-    cd y[LMAX];
-    // forward: y_j = g_j + mu_j y_{j-1}, from zero at the chunk start
-    cd prev = {0.0, 0.0};
-    double Af = 1.0;
-    cd Bf = {0.0, 0.0};
-#pragma unroll
-    for (int m = 0; m < LMAX; ++m) {
-      const int j = j0 + m;
-      if (m < L && j < ny2) {
-        y[m] = Rl(j) + co[5 * j] * prev;
-        prev = y[m];
-        Af = co[5 * j + 3];
-        Bf = y[m];
-      }
-    }
-    // inclusive scan of the maps over the chunks below (lanes p - d)
-#pragma unroll
-    for (int d = 1; d < P; d <<= 1) {
-      const double Au = __shfl_up(Af, d * TC);
-      const cd Bu = {__shfl_up(Bf.x, d * TC), __shfl_up(Bf.y, d * TC)};
-      if (p >= d) {
-        Bf = Af * Bu + Bf;
-        Af = Af * Au;
-      }
-    }
-    cd yin = {__shfl_up(Bf.x, TC), __shfl_up(Bf.y, TC)};
-    if (p == 0) yin = {0.0, 0.0};
-#pragma unroll
-    for (int m = 0; m < LMAX; ++m) {
-      const int j = j0 + m;
-      if (m < L && j < ny2) y[m] = y[m] + co[5 * j + 3] * yin;
-    }
-    // backward: x_j = beta_j y_j + gamma_j x_{j+1}, from zero past the chunk end
-    cd nxt = {0.0, 0.0};
-    double Ab = 1.0;
-    cd Bb = {0.0, 0.0};
-#pragma unroll
-    for (int m = LMAX - 1; m >= 0; --m) {
-      const int j = j0 + m;
-      if (m < L && j < ny2) {
-        y[m] = co[5 * j + 1] * y[m] + co[5 * j + 2] * nxt;
-        nxt = y[m];
-        Ab = co[5 * j + 4];
-        Bb = y[m];
-      }
-    }
-#pragma unroll
-    for (int d = 1; d < P; d <<= 1) {
-      const double Ad = __shfl_down(Ab, d * TC);
-      const cd Bd = {__shfl_down(Bb.x, d * TC), __shfl_down(Bb.y, d * TC)};
-      if (p + d < P) {
-        Bb = Ab * Bd + Bb;
-        Ab = Ab * Ad;
-      }
-    }
-    cd xin = {__shfl_down(Bb.x, TC), __shfl_down(Bb.y, TC)};
-    if (p == P - 1) xin = {0.0, 0.0};
-    const SolveRows& SR = a.rows[e];
-#pragma unroll
-    for (int m = 0; m < LMAX; ++m) {
-      const int j = j0 + m;
-      if (m < L && j < ny2 && act_l && j >= SR.wlo && j <= SR.whi)
-        a.u[e][(long long)j * pc + cl] = y[m] + co[5 * j + 4] * xin;
-    }
-  }
-}
-
-// rem_div_chan (for/solver.f90:1302-1379, BC rows 2330-2371): Poisson rows 1..Nyp
-// by PCR with per-column coefficients, velocity correction, and with
-// update_p the pressure update of rk_chan_1 (for/solver.f90:1261-1267).
-//
-// Every row is kept with off-diagonals a, c >= 0 and diagonal b <= 0 (the bottom
-// BC row is negated), and stored by its row sum s = a + b + c instead of b: the
-// interior rows sum to exactly -(kx^2 + kz^2) and the BC rows to 0 (or -1 for
-// the Dirichlet row of the (0,0) mode).  A reduction step then forms
-//   s' = s + al s(j-s) + ga s(j+s),   b = s - a - c,
-// sums of terms of one sign (al, ga >= 0), where the usual update
-// b' = b + al c(j-s) + ga a(j+s) cancels almost all of b for the weakly dominant
-// rows of small kx^2 + kz^2 (on a 257-row stretched grid plain PCR lost 3-4
-// digits there against the Thomas sweep; this form stays within 10x of it).
-template <int TC, int NT, int RPT>
-__global__ __launch_bounds__(NT) void k_project(ColArgs a, int update_p) {
-  constexpr int RG = NT / TC;
-  extern __shared__ unsigned char smem[];
-  const Geo& g = a.g;
-  const int ny2 = g.ny2, ny = g.ny, tid = threadIdx.x;
-  const int cc = tid % TC, rg = tid / TC;
-  const int tile = xcd_tile(blockIdx.x, (int)(g.pc / TC));
-  if (tile < 0) return;
-  const int c = tile * TC + cc;
-  const int i = c % g.kxp, k = c / g.kxp;
-  const bool active = i < g.kxr;
-  const long long pc = g.pc;
-  cd* sD = (cd*)smem;
-  double* sA = (double*)(sD + TC * ny2);
-  double* sS = sA + TC * ny2;  // row sums a + b + c
-  double* sC = sS + TC * ny2;
-  cd* __restrict__ u1 = a.u[0];
-  cd* __restrict__ u2 = a.u[1];
-  cd* __restrict__ u3 = a.u[2];
-  const double kxi = active ? a.kx[i] : 0.0, kzk = a.kz[k];
-  const double k2 = -(kxi * kxi) - kzk * kzk;
-  // the velocity of the thread's rows, read once for the divergence and kept for
-  // the correction, on the tall columns (at 512x257x512 the second read came
-  // back from HBM: 0.763 -> 0.712 ms); at 3 rows per thread the 56 more VGPRs
-  // cost more occupancy than the reads (256x129x256: 0.084 -> 0.090 ms)
-  constexpr bool KEEP = RPT >= 4 && RPT <= 8;
-  cd ku1[KEEP ? RPT : 1], ku2[KEEP ? RPT : 1], ku3[KEEP ? RPT : 1];
-#pragma unroll
-  for (int m = 0; m < RPT; ++m) {
-    const int j = rg + m * RG;
-    if (j >= ny2) break;
-    const int q = j * TC + cc;
-    double aj = 0.0, sj = 1.0, cj = 0.0;
-    cd d = {0.0, 0.0};
-    if (j == 1) {
-      // (1, -1) Neumann, or (1) for phi(1) = 0 in the (0,0) mode; negated
-      cj = (c == 0) ? 0.0 : 1.0;
-      sj = (c == 0) ? -1.0 : 0.0;
-    } else if (j == ny) {
-      aj = 1.0; sj = 0.0;  // (1, -1)
-    } else if (j > 1 && j < ny) {
-      aj = 1.0 / (a.dy[j] * a.dyf[j]);
-      sj = k2;
-      cj = 1.0 / (a.dy[j + 1] * a.dyf[j]);
-      if (active) {
-        const long long o = (long long)j * pc + c;
-        if (a.prhs) {
-          // poisson_p_chan (for/solver.f90:1382-1560): vec = -(source + the scalars'
-          // y gradient, except in the (0, 0) mode)
-          cd sv = a.prhs[o];
-          if (c != 0)
-            for (int n = 0; n < a.pnth; ++n) {
-              const cd dt = a.u[3 + n][o + pc] - a.u[3 + n][o - pc];
-              const double den = a.gyf[j + 1] - a.gyf[j - 1];
-              sv = sv + cd{dt.x / den, dt.y / den};
-            }
-          d = -1.0 * sv;
-        } else {
-          const cd v1 = u1[o], v2 = u2[o], v3 = u3[o];
-          d = ik(kxi, v1) + (1.0 / a.dyf[j]) * (u2[o + pc] - v2) + ik(kzk, v3);
-          if constexpr (KEEP) { ku1[m] = v1; ku2[m] = v2; ku3[m] = v3; }
-        }
-      }
-    }
-    sA[q] = aj; sS[q] = sj; sC[q] = cj; sD[q] = d;
-  }
-  __syncthreads();
-  for (int l = 0; l < a.plevels; ++l) {
-    const int s = 1 << l;
-    double na[RPT], ns[RPT], nc[RPT];
-    cd nd[RPT];
-#pragma unroll
-    for (int m = 0; m < RPT; ++m) {
-      const int j = rg + m * RG;
-      if (j >= 1 && j <= ny) {
-        const int q = j * TC + cc, qm = q - s * TC, qp = q + s * TC;
-        const int jm = j - s, jp = j + s;
-        double a2 = 0.0, c2 = 0.0, s2 = sS[q];
-        cd d2 = sD[q];
-        if (jm >= 1) {
-          const double bm = sS[qm] - sA[qm] - sC[qm];
-          const double al = -sA[q] / bm;
-          a2 = al * sA[qm];
-          s2 = s2 + al * sS[qm];
-          d2 = d2 + al * sD[qm];
-        }
-        if (jp <= ny) {
-          const double bp = sS[qp] - sA[qp] - sC[qp];
-          const double ga = -sC[q] / bp;
-          c2 = ga * sC[qp];
-          s2 = s2 + ga * sS[qp];
-          d2 = d2 + ga * sD[qp];
-        }
-        na[m] = a2; ns[m] = s2; nc[m] = c2; nd[m] = d2;
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int m = 0; m < RPT; ++m) {
-      const int j = rg + m * RG;
-      if (j >= 1 && j <= ny) {
-        const int q = j * TC + cc;
-        sA[q] = na[m]; sS[q] = ns[m]; sC[q] = nc[m]; sD[q] = nd[m];
-      }
-    }
-    __syncthreads();
-  }
-  for (int m = 0; m < RPT; ++m) {
-    const int j = rg + m * RG;
-    if (j >= ny2) break;
-    const int q = j * TC + cc;
-    sD[q] = (j >= 1 && j <= ny) ? (1.0 / (sS[q] - sA[q] - sC[q])) * sD[q] : cd{0.0, 0.0};
-  }
-  __syncthreads();
-  if (!active) return;
-#pragma unroll
-  for (int m = 0; m < RPT; ++m) {
-    const int j = rg + m * RG;
-    if (j >= ny2) break;
-    if (j < 1 || j > ny) continue;
-    const long long o = (long long)j * pc + c;
-    const cd phi = sD[j * TC + cc];
-    if (a.prhs) {  // cp(j) = vec(j), j = 1..Nyp
-      a.p[o] = phi;
-      continue;
-    }
-    // rows 1 and Nyp were not read above: their divergence row is a BC row
-    const bool kept = KEEP && j > 1 && j < ny;
-    const cd v1 = kept ? ku1[KEEP ? m : 0] : u1[o];
-    const cd v2 = kept ? ku2[KEEP ? m : 0] : u2[o];
-    const cd v3 = kept ? ku3[KEEP ? m : 0] : u3[o];
-    u1[o] = v1 - ik(kxi, phi);
-    u3[o] = v3 - ik(kzk, phi);
-    if (j >= 2) u2[o] = v2 - (1.0 / a.dy[j]) * (phi - sD[(j - 1) * TC + cc]);
-    if (update_p && j >= a.jstart && j <= a.jend) a.p[o] = a.p[o] + (1.0 / a.temp4) * phi;
   }
 }
 

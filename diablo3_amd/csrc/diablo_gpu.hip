@@ -1,13 +1,13 @@
 // diablo_gpu.hip — C ABI of the MI355X RKW3 + Crank–Nicolson channel step.
 //
-// One DNS substep (rk_chan_1, for/solver.f90:366-1273) is five launches:
+// One DNS substep (rk_chan_1, for/solver.f90:366-1273) is four launches:
 //   k_inv_z     packed Fourier state -> x-spectra per z row (z inverse transform)
-//   k_xprod     x inverse transform, nonlinear products with their y stencils,
-//               x forward transform, ikx factors (physical space stays in LDS)
+//   k_xmarch    x inverse transform, nonlinear products with their y stencils,
+//               x forward transform, ikx factors (physical space stays on chip)
 //   k_fwdz_nl   z forward transform of the products -> nonlinear tendencies
-//   k_cn        per (kx,kz) column: Fourier-space assembly of cf (RK memory) and
-//               cr (right-hand side incl. explicit CN half), then the CN solves
-//   k_project   per (kx,kz) column: rem_div_chan and the pressure update
+//   k_column    per (kx,kz) column: Fourier-space assembly of cf (RK memory) and
+//               cr (right-hand side incl. explicit CN half), the CN solves,
+//               rem_div_chan and the pressure update
 // The CN operator of DNS is independent of x and z, so solving it per Fourier
 // column is the same linear map as the reference's per-physical-column solve
 // followed by the forward transform; it saves the 8 transforms the reference
@@ -17,6 +17,7 @@
 #include "../../include/diablo_gpu.h"
 #include "../../include/dgpu_closure.h"
 #include "dgpu_kernels.hpp"
+#include "dgpu_column.hpp"
 #include "dgpu_les.hpp"
 #include "dgpu_closure.hpp"
 #include "dgpu_stats.hpp"
@@ -92,8 +93,6 @@ struct dgpu_handle {
   void* HinZD[MAXF] = {};
   void* PgD[3 * MAXF] = {};
   void* Hout[MAXO] = {};
-  // persistent kernels: blocks to launch (a few per CU)
-  int resident_blocks = 1024;
   void* d_box = nullptr;  // dgpu_box_filter: y weights, row ranges, output
   size_t box_bytes = 0;
   int cus = 256;        // compute units of the device
@@ -212,6 +211,18 @@ __global__ void k_unpack_four(const cd* __restrict__ comp, cd* __restrict__ fort
   }
 }
 
+// filter_chan (for/solver.f90:1597-1685): the horizontal filter of one scalar,
+// cth *= sigma(kx, kz) on rows [jlo, jhi]; sigma [kzr][kxp] from the host
+__global__ __launch_bounds__(256) void k_filter_th(Geo g, cd* __restrict__ th, const double* __restrict__ sigma,
+                                                     int jlo, int jhi) {
+  const long long c = (long long)blockIdx.x * 256 + threadIdx.x;
+  const int j = jlo + blockIdx.y;
+  if (c >= g.pc || j > jhi) return;
+  if (c % g.kxp >= g.kxr) return;
+  const long long o = (long long)j * g.pc + c;
+  th[o] = sigma[c] * th[o];
+}
+
 size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 
 int dalloc(dgpu_handle* h, void** p, size_t bytes) {
@@ -272,26 +283,16 @@ void cn_matrix(const dgpu_handle* h, int F, double temp1, std::vector<double>& a
   }
 }
 
-int pcr_levels(int n) {
-  int l = 0;
-  while ((1 << l) < n) ++l;
-  return l;
-}
-
-struct ColShape;
-int cn_chunk(const dgpu_handle* h);
-
 // Thomas factorisation of one tridiagonal system (rows 0..n-1, a[0] = c[n-1] = 0)
-// for the chunked solve of k_cn: per row j, out[5j..5j+4] = mu_j, beta_j, gamma_j,
-// F_j, G_j with (thomas_forward/backward_real_mpi, for/solver.f90:1691-1852)
+// for the chunked solve of k_column: out[j] = mu_j, out[n + j] = beta_j, out[2n + j] =
+// gamma_j with (thomas_forward/backward_real_mpi, for/solver.f90:1691-1852)
 //   b'_0 = b_0, mu_j = -a_j / b'_{j-1}, b'_j = b_j + mu_j c_{j-1},
 //   forward y_j = g_j + mu_j y_{j-1}, backward x_j = beta_j y_j + gamma_j x_{j+1},
-//   beta_j = 1/b'_j, gamma_j = -c_j/b'_j,
-// and, for chunks of L rows, F_j = prod of mu over [chunk start, j] and G_j = prod
-// of gamma over [j, chunk end].  Long double, stored as double; self-checked by
-// running the chunked algorithm against a long-double Thomas solve.
+//   beta_j = 1/b'_j, gamma_j = -c_j/b'_j.
+// Long double, stored as double; self-checked by running the algorithm of the P
+// chunks of chunk_start against a long-double Thomas solve.
 int thomas_chunk_coefficients(const std::vector<double>& a, const std::vector<double>& b,
-                              const std::vector<double>& c, int L, double* out) {
+                              const std::vector<double>& c, int P, double* out) {
   const int n = (int)b.size();
   std::vector<long double> mu(n), bp(n), be(n), ga(n);
   bp[0] = b[0];
@@ -305,67 +306,61 @@ int thomas_chunk_coefficients(const std::vector<double>& a, const std::vector<do
     if (bp[j] == 0) return fail(20, "singular Crank-Nicolson system");
     be[j] = 1.0L / bp[j];
     ga[j] = -(long double)c[j] / bp[j];
-  }
-  for (int j = 0; j < n; ++j) {
-    const int s0 = j / L * L, e0 = std::min(s0 + L, n) - 1;
-    long double F = 1, G = 1;
-    for (int i = s0; i <= j; ++i) F *= mu[i];
-    for (int i = j; i <= e0; ++i) G *= ga[i];
-    out[5 * j + 0] = (double)mu[j];
-    out[5 * j + 1] = (double)be[j];
-    out[5 * j + 2] = (double)ga[j];
-    out[5 * j + 3] = (double)F;
-    out[5 * j + 4] = (double)G;
+    out[j] = (double)mu[j];
+    out[n + j] = (double)be[j];
+    out[2 * n + j] = (double)ga[j];
   }
   // self-check: the chunked algorithm in double against a long-double Thomas solve
-  std::vector<double> d(n), yl(n);
+  std::vector<double> d(n), yl(n), xl(n);
   std::vector<long double> g(n), x(n);
   for (int j = 0; j < n; ++j) d[j] = std::sin(0.37 * j + 0.1) + 0.5;
   g[0] = d[0];
   for (int j = 1; j < n; ++j) g[j] = d[j] + mu[j] * g[j - 1];
   x[n - 1] = g[n - 1] * be[n - 1];
   for (int j = n - 2; j >= 0; --j) x[j] = be[j] * g[j] + ga[j] * x[j + 1];
-  const int P = (n + L - 1) / L;
-  std::vector<double> yin(P + 1, 0.0), xin(P + 1, 0.0);
-  for (int q = 0; q < P; ++q) {  // forward: local + carries in chunk order
+  double yin = 0.0, xin = 0.0;
+  for (int q = 0; q < P; ++q) {  // forward: from zero at the chunk start, then the carry
+    const int s0 = chunk_start(n, P, q), e0 = chunk_start(n, P, q + 1) - 1;
     double pr = 0.0;
-    for (int j = q * L; j < std::min((q + 1) * L, n); ++j) { yl[j] = d[j] + out[5 * j] * pr; pr = yl[j]; }
-    const int e0 = std::min((q + 1) * L, n) - 1;
-    yin[q + 1] = yl[e0] + out[5 * e0 + 3] * yin[q];
-  }
-  for (int j = 0; j < n; ++j) yl[j] = yl[j] + out[5 * j + 3] * yin[j / L];
-  std::vector<double> xl(n);
-  for (int q = P - 1; q >= 0; --q) {
-    double nx = 0.0;
-    const int s0 = q * L, e0 = std::min((q + 1) * L, n) - 1;
-    for (int j = e0; j >= s0; --j) { xl[j] = out[5 * j + 1] * yl[j] + out[5 * j + 2] * nx; nx = xl[j]; }
-    xin[q] = xl[s0] + out[5 * s0 + 4] * xin[q + 1];
+    for (int j = s0; j <= e0; ++j) pr = yl[j] = d[j] + out[j] * pr;
+    for (int j = s0; j <= e0; ++j) yl[j] = yl[j] + (yin = out[j] * yin);
+    if (e0 >= s0) yin = yl[e0];
   }
   long double err = 0, nrm = 0;
-  for (int j = 0; j < n; ++j) {
-    const long double v = xl[j] + out[5 * j + 4] * xin[j / L + 1];
-    err = std::max(err, std::fabs(v - x[j]));
-    nrm = std::max(nrm, std::fabs(x[j]));
+  for (int q = P - 1; q >= 0; --q) {
+    const int s0 = chunk_start(n, P, q), e0 = chunk_start(n, P, q + 1) - 1;
+    double nx = 0.0;
+    for (int j = e0; j >= s0; --j) nx = xl[j] = out[n + j] * yl[j] + out[2 * n + j] * nx;
+    for (int j = e0; j >= s0; --j) {
+      xl[j] = xl[j] + (xin = out[2 * n + j] * xin);
+      err = std::max(err, std::fabs((long double)xl[j] - x[j]));
+      nrm = std::max(nrm, std::fabs(x[j]));
+    }
+    if (e0 >= s0) xin = xl[s0];
   }
   if (!(err <= 1e-12L * (nrm > 0 ? nrm : 1.0L))) return fail(21, "chunked Thomas disagrees with Thomas");
   return 0;
 }
 
+// The step takes columns of at most 80 KiB of right-hand sides (16 (3 + N_th)
+// bytes a row); taller ones are refused.
+bool column_rows_ok(const dgpu_handle* h) { return (size_t)h->g.ny2 * 16 * (3 + h->nth) <= 80 * 1024; }
+
 int ensure_factors(dgpu_handle* h, double delta_t) {
   if (h->fac_dt == delta_t) return 0;
   const int n2 = h->c.ny + 2, nf = 3 + h->nth;
-  const size_t per_field = (size_t)5 * n2;
+  const size_t per_field = (size_t)3 * n2;
   std::vector<double> buf((size_t)3 * MAXF * per_field, 0.0), a, b, cc;
   const double hb[3] = {delta_t * (8.0 / 15.0), delta_t * (2.0 / 15.0), delta_t * (5.0 / 15.0)};
-  const int L = cn_chunk(h);
-  if (L <= 0) return fail(2, "ny too large for the column kernels");
+  ColShape cs{};
+  if (!column_rows_ok(h) || !column_shape(h->g, &cs)) return fail(2, "ny too large for the column kernels");
   for (int r = 0; r < 3; ++r) {
     const double temp1 = 0.5 * h->c.nu * hb[r];
     for (int F = 0; F < nf; ++F) {
       cn_matrix(h, F, temp1, a, b, cc);
       a[0] = 0.0;
       cc[n2 - 1] = 0.0;
-      int rc = thomas_chunk_coefficients(a, b, cc, L, &buf[((size_t)r * MAXF + F) * per_field]);
+      int rc = thomas_chunk_coefficients(a, b, cc, cs.P, &buf[((size_t)r * MAXF + F) * per_field]);
       if (rc) return rc;
     }
   }
@@ -449,10 +444,10 @@ int ensure_fft_scratch(dgpu_handle* h) {
 // --------------------------------------------------------------------------------
 // per-kernel timing
 // --------------------------------------------------------------------------------
-constexpr int NKERN = 12;
+constexpr int NKERN = 13;
 const char* const kKernelNames[NKERN] = {"k_inv_z",   "k_xprod",  "k_fwdz_nl", "k_cn",      "k_project",
                                          "k_bc_post", "les_grad", "k_amd",     "k_cn_phys", "les_cn_fft",
-                                         "k_closure", "k_xmarch"};
+                                         "k_closure", "k_xmarch", "k_column"};
 
 hipEvent_t pool_event(dgpu_handle* h) {
   if (!h->ev_pool.empty()) {
@@ -675,112 +670,10 @@ int launch_fwdz_nl(dgpu_handle* h, NlArgs& a, int nj) {
   return 0;
 }
 
-// columns per block (TC) and rows per thread (RPT) of the column kernels: the
-// largest TC whose LDS lets at least two blocks share a CU (<= 80 KiB)
-struct ColShape {
-  int tc, rpt;
-  size_t lds;
-};
-ColShape col_shape(const dgpu_handle* h, bool cn) {
-  const int ny2 = h->g.ny2, nf = 3 + h->nth;
-  ColShape cs{};
-  if (cn) {
-    // k_cn: TC columns x all fields in LDS; one wave solves one field of the TC
-    // columns in 64/TC chunks of L <= 32 rows (LMAX = 4 RPT >= L); the widest TC
-    // that fits and still gives the CUs 1.5 blocks each, else the narrowest that fits
-    // (measured on MI355X: at 64x65x64, 946 columns, 8 columns per block 0.0228 ms,
-    // 4 0.0184, 2 0.0160, 1 0.0231; at 256x129x256, 8 0.196, 4 0.243)
-    for (int tc : {8, 4, 2, 1}) {
-      const size_t lds = (size_t)tc * ny2 * 16 * nf;
-      const int rg = 256 / tc, need = (ny2 + rg - 1) / rg;
-      // exact rows per thread for 8 columns (the chunk bound LMAX = 4 RPT then
-      // tracks the column: fewer unrolled Thomas steps), powers of two otherwise
-      int rpt = 1;
-      while (rpt < need) rpt *= 2;
-      if (tc == 8 && need >= 1 && need <= 8) rpt = need;
-      if (lds <= 80 * 1024 && rpt <= 8 && h->g.pc % tc == 0) {
-        cs = {tc, rpt, lds};
-        if (2 * (h->g.pc / tc) >= 3 * h->cus) break;
-      }
-    }
-    return cs;
-  }
-  // k_project: 4 columns per block where that still gives two blocks per CU, else
-  // 2 (measured on MI355X: at 256x129x256, 4 columns 0.080 ms, 2 0.093, 8 0.106;
-  // at 64x65x64, 946 columns, 2 columns 0.011 ms, 4 0.013)
-  const long long want = h->resident_blocks > 0 ? h->resident_blocks : 512;
-  const int tc0 = h->g.pc / 4 >= want ? 4 : 2;
-  for (int tc : {tc0, 2}) {
-    const size_t lds = (size_t)tc * ny2 * 40;
-    if (lds <= 80 * 1024 || (tc == 2 && lds <= 160 * 1024)) {
-      const int rg = 256 / tc, need = (ny2 + rg - 1) / rg;
-      const int rpt = need <= 8 ? need : 16;
-      cs = {tc, rpt, lds};
-      break;
-    }
-  }
-  return cs;
-}
-
-// rows per chunk of the k_cn solve (0 if no shape fits)
-int cn_chunk(const dgpu_handle* h) {
-  const ColShape cs = col_shape(h, true);
-  if (cs.tc == 0) return 0;
-  const int P = 64 / cs.tc;
-  return (h->g.ny2 + P - 1) / P;
-}
-
-int grid_xcd(long long tiles) { return (int)((tiles + 7) / 8 * 8); }
-
-template <typename T, int NTH, int TC, int RPT>
-int launch_cn_t(dgpu_handle* h, ColArgs& a, size_t lds) {
-  constexpr int LMAX = 4 * RPT;
-  if (a.chunk > LMAX || a.chunk * (64 / TC) < h->g.ny2) return fail(2, "column chunking mismatch");
-  HIPCHK(hipFuncSetAttribute((const void*)&k_cn<T, TC, 256, RPT, NTH, LMAX>,
-                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  k_cn<T, TC, 256, RPT, NTH, LMAX><<<grid_xcd(h->g.pc / TC), 256, lds, h->st>>>(a);
-  HIPCHK(hipGetLastError());
-  return 0;
-}
-
-template <int TC, int RPT>
-int launch_project_t(dgpu_handle* h, ColArgs& a, size_t lds, int update_p) {
-  HIPCHK(hipFuncSetAttribute((const void*)&k_project<TC, 256, RPT>,
-                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  k_project<TC, 256, RPT><<<grid_xcd(h->g.pc / TC), 256, lds, h->st>>>(a, update_p);
-  HIPCHK(hipGetLastError());
-  return 0;
-}
-
-// k_project shapes: every rows-per-thread count up to 8 (a power-of-two round-up
-// would leave up to 3 of 8 row slots idle in every PCR level), then 16 for TC = 2
-#define DG_SHAPES(X) X(8, 1) X(8, 2) X(8, 3) X(8, 4) X(8, 5) X(8, 6) X(8, 7) X(8, 8) \
-                     X(4, 1) X(4, 2) X(4, 3) X(4, 4) X(4, 5) X(4, 6) X(4, 7) X(4, 8) \
-                     X(2, 1) X(2, 2) X(2, 3) X(2, 4) X(2, 5) X(2, 6) X(2, 7) X(2, 8) X(2, 16)
-
-#define DG_CN_SHAPES(X) X(8, 1) X(8, 2) X(8, 3) X(8, 4) X(8, 5) X(8, 6) X(8, 7) X(8, 8) \
-                        X(4, 1) X(4, 2) X(4, 4) X(4, 8) \
-                        X(2, 1) X(2, 2) X(2, 4) X(2, 8) X(1, 1) X(1, 2) X(1, 4) X(1, 8)
-
-template <typename T, int NTH>
-int launch_cn(dgpu_handle* h, ColArgs& a) {
-  const ColShape cs = col_shape(h, true);
-  if (cs.tc == 0 || h->g.pc % cs.tc) return fail(2, "ny too large for the column kernels");
-#define DG_X(TC_, RPT_) \
-  if (cs.tc == TC_ && cs.rpt == RPT_) return launch_cn_t<T, NTH, TC_, RPT_>(h, a, cs.lds);
-  DG_CN_SHAPES(DG_X)
-#undef DG_X
-  return fail(2, "ny too large for the column kernels");
-}
-
 int launch_project(dgpu_handle* h, ColArgs& a, int update_p) {
-  const ColShape cs = col_shape(h, false);
-  if (cs.tc == 0 || h->g.pc % cs.tc) return fail(2, "ny too large for the column kernels");
-#define DG_X(TC_, RPT_) \
-  if (cs.tc == TC_ && cs.rpt == RPT_) return launch_project_t<TC_, RPT_>(h, a, cs.lds, update_p);
-  DG_SHAPES(DG_X)
-#undef DG_X
-  return fail(2, "ny too large for the column kernels");
+  ColShape cs{};
+  if (!column_shape(h->g, &cs)) return fail(2, "ny too large for the column kernels");
+  return dgpu::launch_project(a, cs, update_p, h->st);
 }
 
 template <typename F>
@@ -871,7 +764,6 @@ int download_field(dgpu_handle* h, const cd* dev, double* fort) {
 void fill_col_args(dgpu_handle* h, ColArgs& ca, double time) {
   const dgpu_config& c = h->c;
   ca.g = h->g;
-  ca.plevels = pcr_levels(h->g.ny);
   ca.jstart = c.jstart; ca.jend = c.jend;
   for (int n = 0; n < MAXTH; ++n) {
     ca.jstart_th[n] = c.jstart_th[n]; ca.jend_th[n] = c.jend_th[n];
@@ -883,14 +775,23 @@ void fill_col_args(dgpu_handle* h, ColArgs& ca, double time) {
   ca.px0 = c.px0; ca.omega0 = c.omega0; ca.amp_omega0 = c.amp_omega0; ca.time = time;
   ca.temp4 = 1.0;
   ca.cori = c.ro_inv / c.delta;
+  const bool tw = c.flavor_front && c.ro_inv != 0.0;
+  ca.twon = tw ? 1.0 : 0.0;
+  ca.twu_x = ca.twu_z = 0.0;
   for (int n = 0; n < MAXTH; ++n) {
-    ca.twu_x[n] = (c.ro_inv != 0.0 && n < h->nth) ? c.dthdx[n] * c.delta / c.ro_inv : 0.0;
-    ca.twu_z[n] = (c.ro_inv != 0.0 && n < h->nth) ? -1.0 * c.dthdz[n] * c.delta / c.ro_inv : 0.0;
+    if (tw && n < h->nth) {
+      ca.twu_x += c.dthdx[n] * c.delta / c.ro_inv;
+      ca.twu_z += -1.0 * c.dthdz[n] * c.delta / c.ro_inv;
+    }
     ca.nupr[n] = n < h->nth ? c.nu / c.pr[n] : 0.0;
   }
   ca.rowc = h->d_rowc;
   ca.dy = h->d_dy; ca.dyf = h->d_dyf; ca.gy = h->d_gy; ca.gyf = h->d_gyf; ca.kx = h->d_kx; ca.kz = h->d_kz;
   solve_rows(h, time, ca.rows);
+  ca.bcmask = 0;
+  for (int f = 0; f < 3 + h->nth; ++f)
+    for (int s = 0; s < 5; ++s)
+      if (ca.rows[f].kind[s] >= 0) ca.bcmask |= 1ull << (s * MAXF + f);
   for (int f = 0; f < 3 + h->nth; ++f) { ca.u[f] = h->U[f]; ca.cf[f] = h->CF[f]; ca.nl[f] = h->NL[f]; }
   ca.p = h->P;
 }
@@ -1151,12 +1052,10 @@ int substep_les(dgpu_handle* h, int rk, double delta_t, double time, int time_st
   // 5. Fourier assembly of cf and of the right-hand side (molecular explicit half included)
   ColArgs ca{};
   fill_col_args(h, ca, time);
-  ca.rk = rk; ca.do_cn = 0;
+  ca.rk = rk;
   ca.temp1 = temp1; ca.temp3 = temp3; ca.temp4 = temp4; ca.temp5 = temp5;
   ca.t1v = temp1 * c.nu_v_scale;
   for (int n = 0; n < NTH; ++n) ca.t1pr[n] = temp1 / c.pr[n] * c.nu_v_scale;
-  ca.thc = h->d_fac + (size_t)r * MAXF * 5 * g.ny2;
-  ca.chunk = cn_chunk(h);
   // the mixed handle solves for the increment of the state in float transforms,
   // except where courant needs the new velocity in FP64 (rk 3 of an update step)
   const bool courant_now = h->variable_dt && rk == 3 && time_step % h->update_dt == 0;
@@ -1316,21 +1215,21 @@ int substep(dgpu_handle* h, int rk, double delta_t, double time, int time_step, 
   // 4. columns: assembly, CN, projection, pressure
   ColArgs ca{};
   fill_col_args(h, ca, time);
-  ca.rk = rk; ca.do_cn = 1;
+  ca.rk = rk;
   ca.temp1 = temp1; ca.temp3 = temp3; ca.temp4 = temp4; ca.temp5 = temp5;
   ca.t1v = temp1 * c.nu_v_scale;
   for (int n = 0; n < h->nth; ++n) ca.t1pr[n] = temp1 / c.pr[n] * c.nu_v_scale;
-  ca.thc = h->d_fac + (size_t)r * MAXF * 5 * g.ny2;
-  ca.chunk = cn_chunk(h);
-  if ((rc = tbeg(h, 3))) return rc;
-  rc = by_nth(h->nth, [&](auto NTHc) {
-    constexpr int NTH = decltype(NTHc)::value;
-    return mixed ? launch_cn<float, NTH>(h, ca) : launch_cn<double, NTH>(h, ca);
-  });
+  ca.thc = h->d_fac + (size_t)r * MAXF * 3 * g.ny2;
+  ColShape cs{};
+  if (!column_shape(g, &cs)) return fail(2, "ny too large for the column kernels");
+  // courant reads the new velocity before the projection (for/solver.f90:1241-1244):
+  // the column pass stops after the solves then, and the projection follows it
+  const bool courant_now = h->variable_dt && rk == 3 && time_step % h->update_dt == 0;
+  if ((rc = tbeg(h, courant_now ? 3 : 12))) return rc;
+  rc = launch_column(ca, cs, h->nth, mixed, courant_now ? 0 : 1, h->st);
   if (rc || (rc = tend(h))) return rc;
-  // courant on the new velocity, before the projection (for/solver.f90:1241-1244)
-  if (h->variable_dt && rk == 3 && time_step % h->update_dt == 0)
-    if ((rc = courant_dns(h))) return rc;
+  if (!courant_now) return 0;
+  if ((rc = courant_dns(h))) return rc;
   if ((rc = tbeg(h, 4))) return rc;
   if ((rc = launch_project(h, ca, 1))) return rc;
   return tend(h);
@@ -1400,12 +1299,12 @@ int dgpu_create(const dgpu_config* cfg, dgpu_handle** out) {
     if (hipGetDevice(&dev) != hipSuccess) return bail(fail(10, "hipGetDevice"));
     h->dev = dev;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && ncu > 0)
-      h->resident_blocks = 2 * ncu, h->cus = ncu;
+      h->cus = ncu;
     if ((rc = scratch_address(dev, &h->noalloc))) return bail(rc);
   }
   ALLOC(h->twx64, sizeof(cd) * g.nx); ALLOC(h->twz64, sizeof(cd) * g.nz);
   ALLOC(h->twx32, sizeof(cf) * g.nx); ALLOC(h->twz32, sizeof(cf) * g.nz);
-  ALLOC(h->d_fac, sizeof(double) * 3 * MAXF * 5 * n2);
+  ALLOC(h->d_fac, sizeof(double) * 3 * MAXF * 3 * n2);
   ALLOC(h->d_rowc, sizeof(double) * RC_COUNT * n2);
   if (cfg->use_les) {
     // gradients, eddy viscosity and SGS fields in the transform precision; the
@@ -1453,7 +1352,6 @@ int dgpu_create(const dgpu_config* cfg, dgpu_handle** out) {
     double* r = &rowc[(size_t)j * RC_COUNT];
     const double dy = h->dy[j], dyp = h->dy[j + 1], dyf = h->dyf[j], dyfm = h->dyf[j - 1];
     r[RC_RDY] = 1.0 / dy;
-    r[RC_RDYP] = 1.0 / dyp;
     r[RC_RDYF] = 1.0 / dyf;
     r[RC_RDYFM] = 1.0 / dyfm;
     r[RC_WTH] = dyfm / (2.0 * dy);
