@@ -48,8 +48,8 @@ __global__ __launch_bounds__(256) void k_box_filter(BoxArgs a) {
     for (int q = 0; q < 13; ++q) sz[q] = 0.0;
     for (int mz = 0; mz <= a.fz; ++mz) {
       const int z = ((zl * a.fz + mz - a.fz / 2) % g.nz + g.nz) % g.nz;
-      const long long row = ((long long)k * g.nz + z) * g.nx;
-      const long long rowp = row + g.pp;  // row k+1 of u2
+      const long long row = pline(g, k, z);
+      const long long rowp = row + g.nx;  // row k+1 of u2
       double sx[13];
       for (int q = 0; q < 13; ++q) sx[q] = 0.0;
       for (int mx = 0; mx <= a.fx; ++mx) {
@@ -75,7 +75,7 @@ __global__ __launch_bounds__(256) void k_box_filter(BoxArgs a) {
     double sz = 0.0;
     for (int mz = 0; mz <= a.fz; ++mz) {
       const int z = ((zl * a.fz + mz - a.fz / 2) % g.nz + g.nz) % g.nz;
-      const long long row = ((long long)k * g.nz + z) * g.nx;
+      const long long row = pline(g, k, z);
       double sx = 0.0;
       for (int mx = 0; mx <= a.fx; ++mx) {
         const int x = ((xl * a.fx + mx - a.fx / 2) % g.nx + g.nx) % g.nx;

@@ -26,7 +26,7 @@ struct ClosureArgs {
   MlpW w;
   int have_net;   // 0: no network set (every point takes the AMD coefficient)
   double nu, gyb; // molecular viscosity, grav_y
-  void* cgy;      // [ny2][pp] outputs at GY (step mode), precision T; sign bit set
+  void* cgy;      // physical-layout outputs at GY (step mode), precision T; sign bit set
   void* kgy;      // where the point took the AMD value
   int feat, jf0;  // feature mode and its first row
   // per-launch constants: -1/(2 C^2), sqrt(2)/nu, 1/dxs, 1/dzs
@@ -132,7 +132,7 @@ __global__ __launch_bounds__(256) void k_closure(ClosureArgs c) {
   xcd_rows(blockIdx.x, (int)((g.pp + 255) / 256), g.ny2, qb, j);
   const long long q0 = (long long)qb * 256 + threadIdx.x;
   const bool live = q0 < g.pp;
-  const long long q = live ? q0 : g.pp - 1;  // every lane takes part in the MFMA tiles
+  const long long qf = live ? q0 : g.pp - 1, q = pcol(g, qf);  // every lane takes part in the MFMA tiles
   const int ny = g.ny;
   AmdIn<T> in;
   load_window<T, 3 * (3 + NTH)>(in, a, j, q);
@@ -201,7 +201,7 @@ __global__ __launch_bounds__(256) void k_closure(ClosureArgs c) {
   __syncthreads();
   if (c.feat) {
     if (on) {
-      const long long s = (long long)(j - c.jf0) * g.pp + q;
+      const long long s = (long long)(j - c.jf0) * g.pp + qf;
 #pragma unroll
       for (int k = 0; k < MLP_INP; ++k) c.X[s * MLP_INP + k] = fe[k];
       const double r2 = sqrt(2.0 * (double)s2);
@@ -214,7 +214,7 @@ __global__ __launch_bounds__(256) void k_closure(ClosureArgs c) {
   }
   if (!live) return;
   // coefficients (1/time) at GY: the network's sqrt(2 s2) max(0, y), or AMD's stored negated
-  const long long o = (long long)j * g.pp + q;
+  const long long o = (long long)j * g.nx + q;
   const float r2 = sqrtf(2.f * s2);
   ((T*)c.cgy)[o] = inside ? (T)(r2 * fmaxf(0.f, sY[wave][lane][0])) : -amd_v;
   ((T*)c.kgy)[o] = inside ? (T)(r2 * fmaxf(0.f, sY[wave][lane][1])) : -amd_t;
@@ -224,12 +224,12 @@ __global__ __launch_bounds__(256) void k_closure(ClosureArgs c) {
 // network: the sign bit of cgy is clear there (k_closure stores the AMD fallback
 // negated).  One atomic per block into count.
 template <typename T>
-__global__ __launch_bounds__(256) void k_closure_count(const T* __restrict__ cgy, long long pp, int ny,
+__global__ __launch_bounds__(256) void k_closure_count(const T* __restrict__ cgy, Geo g,
                                                         unsigned long long* count) {
-  const long long n = (long long)(ny - 1) * pp, base = 2 * pp;
+  const long long n = (long long)(g.ny - 1) * g.pp;
   int c = 0;
   for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256)
-    c += signbit(cgy[base + i]) ? 0 : 1;
+    c += signbit(cgy[pcol(g, i % g.pp) + (2 + i / g.pp) * g.nx]) ? 0 : 1;
   // block sum through LDS
   __shared__ int sc[256];
   sc[threadIdx.x] = c;

@@ -34,12 +34,6 @@
 
 namespace dgpu {
 
-// Rows 0..n-1 in P chunks: base rows each, one more for the last n mod P of them.
-__host__ __device__ inline int chunk_start(int n, int P, int p) {
-  const int base = n / P, rem = n - base * P, extra = p - (P - rem);
-  return p * base + (extra > 0 ? extra : 0);
-}
-
 constexpr int COLUMN_NT = 512;    // threads per block at most: 256 registers per thread
 constexpr int COLUMN_ROWS = 320;  // rows whose tables fit LDS beside the exchange (8 columns, 5 rows a chunk)
 

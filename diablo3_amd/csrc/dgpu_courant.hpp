@@ -29,7 +29,7 @@ __global__ __launch_bounds__(256) void k_courant(CourantArgs a) {
   double m = INFINITY;
   for (long long q = (long long)blockIdx.x * 256 + threadIdx.x; q < npts; q += (long long)gridDim.x * 256) {
     const int j = a.jlo + (int)(q / g.pp);
-    const long long o = (long long)j * g.pp + q % g.pp;
+    const long long o = pcol(g, q % g.pp) + (long long)j * g.nx;
     const double u1 = a.u1[o], u2 = a.u2[o], u3 = a.u3[o];
     if (a.front) {
       for (int n = 0; n < a.nth; ++n) {

@@ -6,7 +6,11 @@
 //                        double), k = 0..2Nkz (kzr), j = 0..ny+1; pc = kxp*kzr.
 //   x-spectra H[j][z][i] complex T: the x transform of physical line (j, z)
 //                        restricted to i = 0..Nkx, same pitch kxp (ph = nz*kxp).
-//   physical R[j][z][x]  T (pp = nz*nx).
+//   physical R[z][j][x]  T (pp = nz*nx points a plane): the y column of a point lies in
+//                        one slab of ny2 nx values, rows nx apart.  The kernels
+//                        that march or solve in y then stay within a page or two;
+//                        with z inside j ([j][z][x]) the rows of a column are nz nx
+//                        values apart, a page each.
 // Padding columns i = kxr..kxp-1 are zero and never read as modes.
 // Every kernel indexes only inside these extents; grids are sized by the host to
 // the same extents (the host checks them before launch).
@@ -22,7 +26,22 @@ constexpr int MAXO = 3 * MAXF;         // largest transform batch (LES: v, dv/dx
 struct Geo {
   int nx, nz, ny, ny2, nkx, nkz, kxr, kzr, kxp;
   long long pc, ph, pp;
+  int lx;  // log2 nx
 };
+// first point of physical line (j, z); a point of plane 0 by its index z nx + x, and
+// the distance from row to row
+__host__ __device__ __forceinline__ long long pline(const Geo& g, int j, int z) {
+  return ((long long)z * g.ny2 + j) * g.nx;
+}
+__device__ __forceinline__ long long pcol(const Geo& g, long long q) {
+  return ((q >> g.lx) * g.ny2 << g.lx) + (q & (g.nx - 1));
+}
+
+// Rows 0..n-1 in P chunks: base rows each, one more for the last n mod P of them.
+__host__ __device__ inline int chunk_start(int n, int P, int p) {
+  const int base = n / P, rem = n - base * P, extra = p - (P - rem);
+  return p * base + (extra > 0 ? extra : 0);
+}
 
 template <typename P, int M>
 struct Ptrs {
@@ -97,10 +116,12 @@ __global__ __launch_bounds__(NT) void k_inv_z(Ptrs<const cd*, MAXO> src, Ptrs<cx
   }
 }
 
-// ACC: add the transform into the destination (an increment of the state)
+// ACC: add the transform into the destination (an increment of the state).
+// dj, dk: distance of the destination's planes and kz rows (the packed layout's, or
+// a Fortran array's, whose columns kxr..izero-1 the plane's last block fills with zeros).
 template <typename T, int NZ, int TI, int NT, bool ACC = false>
-__global__ __launch_bounds__(NT) void k_fwd_z(Ptrs<const cx<T>*, MAXO> src, Ptrs<cd*, MAXO> dst,
-                                              Geo g, int j0, const cx<T>* __restrict__ tw) {
+__global__ __launch_bounds__(NT) void k_fwd_z(Ptrs<const cx<T>*, MAXO> src, Ptrs<cd*, MAXO> dst, Geo g, int j0,
+                                              const cx<T>* __restrict__ tw, long long dj, int dk, int izero) {
   constexpr int LD = NZ + 1;
   __shared__ cx<T> s[TI * LD];
   __shared__ cx<T> stw[NZ];  // twiddles
@@ -116,15 +137,20 @@ __global__ __launch_bounds__(NT) void k_fwd_z(Ptrs<const cx<T>*, MAXO> src, Ptrs
   }
   __syncthreads();
   fft_lds<T, NZ, TI, NT, -1>(s, LD, stw, tid);
-  cd* __restrict__ C = dst.p[f] + (long long)j * g.pc;
+  cd* __restrict__ C = dst.p[f] + j * dj;
   const double rnz = 1.0 / NZ;
   for (int idx = tid; idx < TI * g.kzr; idx += NT) {
     const int ii = idx % TI, p = idx / TI, i = i0 + ii;
     if (i < g.kxr) {
       cd v = cvt<double>(s[ii * LD + swz<T>(zpos(g, p))]);
-      if constexpr (ACC) C[(long long)p * g.kxp + i] = C[(long long)p * g.kxp + i] + rnz * v;
-      else C[(long long)p * g.kxp + i] = rnz * v;
+      cd& c = C[(long long)p * dk + i];
+      if constexpr (ACC) c = c + rnz * v;
+      else c = rnz * v;
     }
+  }
+  if (i0 + TI >= g.kxr) {
+    const int nzc = izero - g.kxr;
+    for (int idx = tid; idx < nzc * g.kzr; idx += NT) C[(long long)(idx / nzc) * dk + g.kxr + idx % nzc] = cd{0.0, 0.0};
   }
 }
 
@@ -212,27 +238,29 @@ __global__ __launch_bounds__(NT) void k_inv_x(Ptrs<const cx<T>*, MAXO> src, Ptrs
   }
   __syncthreads();
   fft_lds_sync<T, NX, ZP, NT, +1>(s, NX, stw, tid);
-  T* __restrict__ R = dst.p[f] + (long long)j * g.pp;
+  T* __restrict__ R = dst.p[f];
   for (int idx = tid; idx < ZP * NX; idx += NT) {
     const int q = idx / NX, n = idx % NX, z = zb + 2 * q;
     const cx<T> v = s[q * NX + swz<T>(n)];
-    R[(long long)z * NX + n] = v.x;
-    R[(long long)(z + 1) * NX + n] = v.y;
+    R[pline(g, j, z) + n] = v.x;
+    R[pline(g, j, z + 1) + n] = v.y;
   }
 }
 
+// sj, sz: distance of the physical lines of consecutive planes and rows (the device
+// layout's, or a Fortran array's).
 template <typename T, int NX, int ZP, int NT>
 __global__ __launch_bounds__(NT) void k_fwd_x(Ptrs<const T*, MAXO> src, Ptrs<cx<T>*, MAXO> dst,
-                                              Geo g, int j0, const cx<T>* __restrict__ tw) {
+                                              Geo g, int j0, const cx<T>* __restrict__ tw, long long sj, long long sz) {
   __shared__ cx<T> s[ZP * NX];
   __shared__ cx<T> stw[NX];  // twiddles
   stage_twiddles<T, NX, NT>(stw, tw, threadIdx.x);
   const int f = blockIdx.z, j = j0 + blockIdx.y, tid = threadIdx.x;
   const int zb = blockIdx.x * ZP * 2;
-  const T* __restrict__ R = src.p[f] + (long long)j * g.pp;
+  const T* __restrict__ R = src.p[f] + j * sj;
   for (int idx = tid; idx < ZP * NX; idx += NT) {
     const int q = idx / NX, n = idx % NX, z = zb + 2 * q;
-    s[q * NX + swz<T>(n)] = {R[(long long)z * NX + n], R[(long long)(z + 1) * NX + n]};
+    s[q * NX + swz<T>(n)] = {R[z * sz + n], R[(z + 1) * sz + n]};
   }
   __syncthreads();
   fft_lds_sync<T, NX, ZP, NT, -1>(s, NX, stw, tid);
@@ -295,7 +323,7 @@ struct XProdArgs {
   // (tau_11, tau_13, tau_33, the two stress fluxes, the two GY stresses, the
   // scalar fluxes); null for DNS
   const void* aug[7 + 2 * MAXTH];
-  // the fields in physical space ([j][z][x], T), all planes, written by the
+  // the fields in physical space ([z][j][x], T), all planes, written by the
   // inverse x transform; the kernel reads the three planes of its x columns
   const void* phys[MAXF];
 };
@@ -427,8 +455,8 @@ __global__ __launch_bounds__(NT) void k_xprod(XProdArgs a) {
   __syncthreads();  // the twiddle table
   // (field f, plane j-1+d) of the line pair (z, z+1) at column x
   auto field = [&](int f, int d, int x) -> cx<T> {
-    const T* R = (const T*)a.phys[f] + (long long)(j - 1 + d) * g.pp + (long long)z * NX + x;
-    return cx<T>{R[0], R[NX]};
+    const T* R = (const T*)a.phys[f] + pline(g, j - 1 + d, z) + x;
+    return cx<T>{R[0], R[(long long)g.ny2 * NX]};
   };
   for (int x = tid; x < NX; x += NT) {
     cx<T> U1[3], U2[3], U3[3];
@@ -446,10 +474,10 @@ __global__ __launch_bounds__(NT) void k_xprod(XProdArgs a) {
     cx<T> P[NP];
     xprod_products<T, NTH>(a, j, U1, U2, U3, TH, P);
     if constexpr (LES) {
-      const long long pz = (long long)j * g.pp + (long long)z * NX + x;
+      const long long pz = pline(g, j, z) + x;
       auto A = [&](int m) {
         const T* p = (const T*)a.aug[m];
-        return cx<T>{p[pz], p[pz + NX]};
+        return cx<T>{p[pz], p[pz + (long long)g.ny2 * NX]};
       };
       P[1] = P[1] + A(0);
       P[0] = P[0] + A(1);

@@ -118,7 +118,7 @@ __global__ __launch_bounds__(256) void k_bc_post(BcArgs a) {
 
 // ---------------------------------------------------------------------------
 // AMD model per point (for/les.f90:571-797, 1213-1346).
-// Inputs (physical, [j][z][x], all planes): for each transported field v in
+// Inputs (physical, [z][j][x], all planes): for each transported field v in
 // (u1, u2, u3, th_n): v, dv/dx, dv/dz.  Outputs, on every plane (zero where the
 // reference adds nothing):
 //   nu_t, kappa_t_n            at GY points, zero at j = 0, 1, 2, Nyp, Nyp+1
@@ -167,7 +167,7 @@ template <typename T>
 struct AmdIn {
   T w[3 * MAXF][4];
   int j0;          // j - 1
-  long long pp;
+  int nx;          // from row to row
   __device__ T at(int f, int row, long long) const { return w[f][row - j0]; }
 };
 // NS slots; rows outside 0..Nyp+1 are clamped (no caller uses such a row's value)
@@ -175,14 +175,14 @@ template <typename T, int NS>
 __device__ __forceinline__ void load_window(AmdIn<T>& in, const AmdArgs& a, int j, long long q) {
   const int last = a.g.ny + 1;
   in.j0 = j - 1;
-  in.pp = a.g.pp;
+  in.nx = a.g.nx;
 #pragma unroll
   for (int s = 0; s < NS; ++s)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       int row = j - 1 + r;
       row = row < 0 ? 0 : (row > last ? last : row);
-      in.w[s][r] = ((const T*)a.f[s])[(long long)row * a.g.pp + q];
+      in.w[s][r] = ((const T*)a.f[s])[(long long)row * a.g.nx + q];
     }
 }
 
@@ -315,8 +315,8 @@ __device__ __forceinline__ T model_gyf(const AmdIn<T>& in, const AmdArgs& a, int
     return coef_gyf(in, a, j, q);
   } else if constexpr (MODEL == 6) {
     // the mean of the network's GY j and j+1 values, else the type-5 GYF coefficient
-    const R c0 = (R)((const T*)a.cgy)[(long long)j * in.pp + q];
-    const R c1 = (R)((const T*)a.cgy)[(long long)(j + 1) * in.pp + q];
+    const R c0 = (R)((const T*)a.cgy)[(long long)j * in.nx + q];
+    const R c1 = (R)((const T*)a.cgy)[(long long)(j + 1) * in.nx + q];
     return (!signbit(c0) && !signbit(c1)) ? R(0.5) * (c0 + c1) : coef_gyf(in, a, j, q);
   } else {
     const Sgyf<T> f = sgyf_plane(in, a, j, q);
@@ -338,7 +338,7 @@ __device__ __forceinline__ T model_gy(const AmdIn<T>& in, const AmdArgs& a, int 
   if constexpr (MODEL == 5) {
     return coef_gy(in, a, j, q);
   } else if constexpr (MODEL == 6) {
-    return fabs((R)((const T*)a.cgy)[(long long)j * in.pp + q]);
+    return fabs((R)((const T*)a.cgy)[(long long)j * in.nx + q]);
   } else {
     const Sgyf<T> f = sgyf_plane(in, a, j, q), fm = sgyf_plane(in, a, j - 1, q);
     const Sgy<T> p = sgy_plane(in, a, j, q);
@@ -445,12 +445,13 @@ __global__ __launch_bounds__(256) void k_amd(AmdArgs a) {
   const Geo& g = a.g;
   int qb, j;
   xcd_rows(blockIdx.x, (int)((g.pp + 255) / 256), g.ny2, qb, j);
-  const long long q = (long long)qb * 256 + threadIdx.x;
-  if (q >= g.pp) return;
+  const long long q0 = (long long)qb * 256 + threadIdx.x;
+  if (q0 >= g.pp) return;
+  const long long q = pcol(g, q0);
   AmdIn<T> in;
   load_window<T, 3 * (3 + NTH)>(in, a, j, q);
   const int ny = g.ny;
-  const long long o = (long long)j * g.pp + q;
+  const long long o = (long long)j * g.nx + q;
   auto put = [&](void* p, R v) { ((T*)p)[o] = (T)v; };
   // the model coefficient at GY j and j + 1, each evaluated once: nu_t, the two
   // stresses at GY j and the GYF flux differences take them (row 1 of types 4
@@ -514,7 +515,7 @@ __global__ __launch_bounds__(256) void k_amd(AmdArgs a) {
     if (j >= a.jstart_th[n] && j <= a.jend_th[n]) {
       R s1;
       if constexpr (MODEL == 6) {
-        const R k0 = (R)((const T*)a.kgy)[o], k1 = (R)((const T*)a.kgy)[o + g.pp];
+        const R k0 = (R)((const T*)a.kgy)[o], k1 = (R)((const T*)a.kgy)[o + g.nx];
         s1 = (!signbit(k0) && !signbit(k1)) ? R(0.5) * (k0 + k1) : amd_th_gyf(in, a, ft, j, q).c;
       } else {
         s1 = amd_th_gyf(in, a, ft, j, q).c;
@@ -525,187 +526,6 @@ __global__ __launch_bounds__(256) void k_amd(AmdArgs a) {
     }
     put(a.aug[7 + 2 * n], fx);
     put(a.aug[8 + 2 * n], fz);
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Crank–Nicolson solve per physical (x, z) column with the eddy viscosity /
-// diffusivity (rk_chan_1, for/solver.f90:875-903, 990-1233): the explicit half
-// of the nu_t term is added to the right-hand side r (the inverse transform of
-// the Fourier right-hand side, which already holds the molecular part), the
-// matrix gets the implicit half, the BC rows of apply_BC_* are set for every
-// column, and Thomas (thomas_forward/backward_real_mpi at one rank,
-// for/solver.f90:1691-1761, 1816-1852) solves rows 0..Nyp+1.
-// One thread per (column, field): the fields' systems are independent, so
-// blockIdx.y picks the field.  The thread keeps a register window of u and nu_t
-// over rows j-1..j+1 and has the loads of the next rows in flight while row j
-// is eliminated (the elimination chain is serial in j; the loads are not).
-// The reciprocal pivot 1/b' and g' go to scratch; the back substitution reads
-// them in reverse with the same look-ahead and recomputes c from nu_t (the
-// same row function, so the same value).
-//
-// INC (the mixed-precision path): u is the state at the substep's start in
-// float and r holds r - u (float).  The solve is then for the increment
-// delta = u_new - u: right-hand side rhs - (l u_{j-1} + d u_j + c u_{j+1}) of the
-// same rows, eliminated in FP64, and delta is written back to r (0 outside
-// [wlo, whi]), so the state moves by a float transform of an O(dt) quantity.
-// The scratch 1/b', g' of the increment system is stored in float (g' is an
-// increment too; the rounding is of the order of the float transforms').
-// Otherwise the solution overwrites u on rows [wlo, whi].
-// ---------------------------------------------------------------------------
-template <typename TU, typename TV>
-struct PhysCnArgs {
-  Geo g;
-  int nf;
-  int field[MAXF];                    // slot -> field (0 u1, 1 u2, 2 u3, 3+n th_n)
-  int blo[MAXF], bhi[MAXF], wlo[MAXF], whi[MAXF];
-  int lo_kind[MAXF], hi_kind[MAXF];   // BC code at each wall (0 Dirichlet, 1 Neumann)
-  double lo_c1[MAXF], hi_c1[MAXF];
-  double tcn[MAXF];                   // temp1 nu_v_scale (/Pr for scalars)
-  double temp2;
-  const double* __restrict__ dy;
-  const double* __restrict__ dyf;
-  const double* __restrict__ rowc;    // [ny2][RC_COUNT] per-row grid coefficients
-  TU* u[MAXF];                        // physical field
-  TU* r[MAXF];                        // right-hand side (INC: r - u, then delta)
-  const TV* visc[MAXF];               // nu_t (velocity) or kappa_t_n (scalar)
-  double* cp;                         // scratch, nf * 2 * ny2 planes: 1/b', g'
-};
-
-template <bool INC>
-struct ScratchType { using type = double; };
-template <>
-struct ScratchType<true> { using type = float; };
-
-template <typename TU, typename TV, bool INC>
-__global__ __launch_bounds__(256) void k_cn_phys(PhysCnArgs<TU, TV> a) {
-  const Geo& g = a.g;
-  const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
-  const int e = blockIdx.y;
-  if (q >= g.pp || e >= a.nf) return;
-  const int ny = g.ny, n2 = g.ny2, last = ny + 1;
-  const long long pp = g.pp;
-  const double* __restrict__ dy = a.dy;
-  const double* __restrict__ dyf = a.dyf;
-  const double* __restrict__ rowc = a.rowc;
-  TU* __restrict__ u = a.u[e];
-  TU* __restrict__ r = a.r[e];
-  const TV* __restrict__ nt = a.visc[e];
-  // scratch: FP64 for the FP64 solve, float for the increments (below)
-  using TS = typename ScratchType<INC>::type;
-  TS* __restrict__ sb = (TS*)a.cp + (long long)e * 2 * n2 * pp;  // 1/b'
-  TS* __restrict__ sg = sb + (long long)n2 * pp;                 // g'
-  const double T = a.tcn[e], t2 = a.temp2;
-  const int fld = a.field[e];
-  const bool v2 = (fld == 1);
-  const int blo = a.blo[e], bhi = a.bhi[e], wlo = a.wlo[e], whi = a.whi[e];
-  // row j of the system: (l, d, c | rhs) from the window values
-  auto row = [&](int j, double um, double uc, double up, double nm, double nc, double np, double rv, double& l,
-                 double& d, double& c, double& rhs) {
-    l = 0.0; d = 1.0; c = 0.0; rhs = 0.0;
-    if (j >= blo && j <= bhi) {
-      rhs = INC ? rv + uc : rv;
-      // The reference's rows (for/solver.f90:1136-1145 and the nu_t terms of
-      // les_chan) divide T and temp2 nu by dy(j) dyf(j) and dy(j+1) dyf(j)
-      // (GYF rows), dyf(j-1) dy(j) and dyf(j) dy(j) (u2's GY rows, nu_t averaged
-      // to the faces); the host table holds those reciprocals, so a row costs
-      // multiplications only (the quotients agree to rounding).
-      const double* k = rowc + (long long)j * RC_COUNT;
-      const double nlo = v2 ? 0.5 * (nc + nm) : nc, nhi = v2 ? 0.5 * (nc + np) : np;
-      const double ilo = k[v2 ? RC_GLO : RC_FLO], ihi = k[v2 ? RC_GHI : RC_FHI];
-      const double lo = (T + t2 * nlo) * ilo, hi = (T + t2 * nhi) * ihi;
-      l = -lo;
-      c = -hi;
-      d = 1.0 + lo + hi;
-      rhs = rhs + t2 * (nhi * (up - uc) * ihi - nlo * (uc - um) * ilo);
-    }
-    // BC rows (apply_BC_* of the reference, for/solver.f90:1901-2232)
-    if (!v2) {
-      if (j == 0) { l = 0.; d = 1.; c = 0.; rhs = 0.; }
-      if (j == 1) {
-        if (a.lo_kind[e] == DGPU_BC_DIRICHLET) { l = 0.; d = 1.; c = 0.; rhs = a.lo_c1[e]; }
-        else { l = 0.; d = -1.; c = 1.; rhs = dy[2] * a.lo_c1[e]; }
-      }
-      if (j == ny) {
-        if (a.hi_kind[e] == DGPU_BC_DIRICHLET) { l = 0.; d = 1.; c = 0.; rhs = a.hi_c1[e]; }
-        else { l = -1.; d = 1.; c = 0.; rhs = dy[ny] * a.hi_c1[e]; }
-      }
-      if (j == ny + 1) { l = 0.; d = 1.; c = 0.; rhs = 0.; }
-    } else {
-      if (a.lo_kind[e] == DGPU_BC_DIRICHLET) {
-        if (j == 1 || j == 2) { l = 0.; d = 1.; c = 0.; rhs = a.lo_c1[e]; }
-      } else if (a.lo_kind[e] == DGPU_BC_NEUMANN) {
-        if (j == 1) { l = 0.; d = -1.; c = 1.; rhs = dyf[1] * a.lo_c1[e]; }
-      }
-      if (j == 0) { l = 0.; d = 1.; c = 0.; rhs = 0.; }
-      if (a.hi_kind[e] == DGPU_BC_DIRICHLET) {
-        if (j == ny + 1 || j == ny) { l = 0.; d = 1.; c = 0.; rhs = a.hi_c1[e]; }
-      } else if (a.hi_kind[e] == DGPU_BC_NEUMANN) {
-        if (j == ny + 1) { l = -1.; d = 1.; c = 0.; rhs = dyf[ny] * a.hi_c1[e]; }
-      }
-    }
-    if (INC) rhs = rhs - (l * um + d * uc + c * up);
-  };
-  // forward elimination; the loads run L + 1 rows (u, nu_t) and L rows (r)
-  // ahead of the elimination, held raw in small register queues (float rows
-  // carry half the bytes per load, so the increment solve keeps more in flight)
-  constexpr int L = INC ? 4 : 2;
-  auto LU = [&](const TU* p, int j) -> TU { return (j >= 0 && j <= last) ? p[(long long)j * pp + q] : (TU)0; };
-  auto LV = [&](int j) -> TV { return (j >= 0 && j <= last) ? nt[(long long)j * pp + q] : (TV)0; };
-  double um = 0.0, uc = (double)LU(u, 0), up = (double)LU(u, 1);
-  double nm = 0.0, nc = (double)LV(0), np = (double)LV(1);
-  double rv = (double)LU(r, 0);
-  TU qu[L], qr[L];
-  TV qv[L];
-#pragma unroll
-  for (int i = 0; i < L; ++i) { qu[i] = LU(u, i + 2); qv[i] = LV(i + 2); qr[i] = LU(r, i + 1); }
-  double binv = 0.0, cprev = 0.0, gprev = 0.0;
-  for (int j = 0; j <= last; ++j) {
-    // here up = u(j+1), qu[i] = u(j+2+i) (nu_t alike), rv = r(j), qr[i] = r(j+1+i)
-    double l, d, c, rhs;
-    row(j, um, uc, up, nm, nc, np, rv, l, d, c, rhs);
-    if (j > 0) {
-      const double m = -l * binv;
-      d = d + m * cprev;
-      rhs = rhs + m * gprev;
-    }
-    binv = 1.0 / d;
-    const long long o = (long long)j * pp + q;
-    sb[o] = (TS)binv;
-    sg[o] = (TS)rhs;
-    cprev = c; gprev = rhs;
-    um = uc; uc = up; up = (double)qu[0];
-    nm = nc; nc = np; np = (double)qv[0];
-    rv = (double)qr[0];
-#pragma unroll
-    for (int i = 0; i < L - 1; ++i) { qu[i] = qu[i + 1]; qv[i] = qv[i + 1]; qr[i] = qr[i + 1]; }
-    qu[L - 1] = LU(u, j + L + 2); qv[L - 1] = LV(j + L + 2); qr[L - 1] = LU(r, j + L + 1);
-  }
-  // back substitution, rows last..0; c of row j from nu_t at j, j+1
-  auto LS = [&](const TS* p, int j) -> TS { return j >= 0 ? p[(long long)j * pp + q] : (TS)0; };
-  auto put = [&](int j, double v) {
-    const long long o = (long long)j * pp + q;
-    if (INC) r[o] = (TU)((j >= wlo && j <= whi) ? v : 0.0);
-    else if (j >= wlo && j <= whi) u[o] = (TU)v;
-  };
-  double x = gprev * binv;
-  put(last, x);
-  double bc = (double)LS(sb, last - 1), gc = (double)LS(sg, last - 1);
-  double vp = (double)LV(last), vc = (double)LV(last - 1);
-  TS qb[L], qg[L];
-#pragma unroll
-  for (int i = 0; i < L; ++i) { qb[i] = LS(sb, last - 2 - i); qg[i] = LS(sg, last - 2 - i); qv[i] = LV(last - 2 - i); }
-  for (int j = last - 1; j >= 0; --j) {
-    // here bc, gc = row j's 1/b', g'; qb[i] = row j-1-i's (nu_t alike: vc = nu(j), vp = nu(j+1))
-    double l, d, c, rhs;
-    row(j, 0.0, 0.0, 0.0, 0.0, vc, vp, 0.0, l, d, c, rhs);
-    x = (gc - c * x) * bc;
-    put(j, x);
-    bc = (double)qb[0]; gc = (double)qg[0];
-    vp = vc; vc = (double)qv[0];
-#pragma unroll
-    for (int i = 0; i < L - 1; ++i) { qb[i] = qb[i + 1]; qg[i] = qg[i + 1]; qv[i] = qv[i + 1]; }
-    qb[L - 1] = LS(sb, j - 1 - L); qg[L - 1] = LS(sg, j - 1 - L); qv[L - 1] = LV(j - 1 - L);
   }
 }
 

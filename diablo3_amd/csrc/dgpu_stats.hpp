@@ -73,8 +73,8 @@ __global__ __launch_bounds__(256) void k_stat_mean(StatArgs a) {
           v = C[(long long)j * g.pc].x;
         }
       } else {
-        const double* __restrict__ F = a.f[fs] + (long long)j * g.pp + x;
-        for (int z = 0; z < g.nz; ++z) v += F[(long long)z * g.nx];
+        const double* __restrict__ F = a.f[fs] + x;
+        for (int z = 0; z < g.nz; ++z) v += F[pline(g, j, z)];
         v = v / (double)g.nz;
       }
     }
@@ -88,11 +88,11 @@ __global__ __launch_bounds__(256) void k_stat_mean(StatArgs a) {
 struct StatPoint {
   const StatArgs& a;
   const int x;
-  const long long pl, pp;
+  const long long pl;
   __device__ StatPoint(const StatArgs& a_, int x_)
-      : a(a_), x(x_), pl((long long)a_.g.ny2 * a_.g.nx), pp(a_.g.pp) {}
+      : a(a_), x(x_), pl((long long)a_.g.ny2 * a_.g.nx) {}
   __device__ double M(int m, int j) const { return a.zm[m * pl + (long long)j * a.g.nx + x]; }
-  __device__ double F(int s, int j, int z) const { return a.f[s][(long long)j * pp + (long long)z * a.g.nx + x]; }
+  __device__ double F(int s, int j, int z) const { return a.f[s][pline(a.g, j, z) + x]; }
   // the dissipation integrand of compute_TKE_diss on GY rows 2..Nyp, zero elsewhere
   // (for/diagnostics.f90:820-1016); when x is not homogeneous the kz = 0 row of
   // each x derivative (k_start = 1), i.e. its z-line mean, is left out
@@ -350,13 +350,13 @@ __global__ __launch_bounds__(256) void k_stat_plane(StatArgs a) {
 // of the sum.  Other rows are zero.
 __global__ __launch_bounds__(256) void k_pp_source(StatArgs a, double* __restrict__ out) {
   const Geo& g = a.g;
-  const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
+  const long long q0 = (long long)blockIdx.x * 256 + threadIdx.x;
   const int j = blockIdx.y;
-  if (q >= g.pp) return;
-  const long long pp = g.pp, o = (long long)j * pp + q;
+  if (q0 >= g.pp) return;
+  const long long q = pcol(g, q0), o = (long long)j * g.nx + q;
   double v = 0.0;
   if (j >= 2 && j <= g.ny) {
-    auto F = [&](int s, int jj) { return a.f[s][(long long)jj * pp + q]; };
+    auto F = [&](int s, int jj) { return a.f[s][(long long)jj * g.nx + q]; };
     const double r2f = 1.0 / (2.0 * a.dyf[j]);
     const double f1 = F(1, j), f2 = (F(3, j + 1) - F(3, j)) / a.dyf[j], f3 = F(8, j);
     const double g1 = (F(0, j + 1) - F(0, j - 1)) * r2f, g2 = 0.5 * (F(4, j) + F(4, j + 1));
@@ -504,7 +504,7 @@ __global__ __launch_bounds__(256) void k_stat_xz(StatArgs a, double* __restrict_
 // integrand, zero on row 1), omega_x, omega_y, omega_z, then th_n.
 struct MovieArgs {
   int nxm, nym, nzm, nfld;
-  const void* nut;  // [j][z][x] in the handle's precision (null: zeros)
+  const void* nut;  // [z][j][x] in the handle's precision (null: zeros)
   int nut_f32;
   double* out;
 };
@@ -521,7 +521,7 @@ __global__ __launch_bounds__(256) void k_stat_movie(StatArgs a, MovieArgs m) {
   else if (t < n1 + n2) { if (m.nym < 1) return; z = (int)((t - n1) / nx); x = (int)((t - n1) % nx); j = m.nym; }
   else { j = (int)((t - n1 - n2) / nz) + 1; z = (int)((t - n1 - n2) % nz); x = m.nxm; }
   const StatPoint P(a, x);
-  const long long pt = (long long)j * g.pp + (long long)z * nx + x;
+  const long long pt = pline(g, j, z) + x;
   double ox, oy, oz;
   P.omega(j, z, ox, oy, oz);
   double nt = 0.0;

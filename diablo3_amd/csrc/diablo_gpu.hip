@@ -19,6 +19,7 @@
 #include "dgpu_kernels.hpp"
 #include "dgpu_column.hpp"
 #include "dgpu_les.hpp"
+#include "dgpu_cn_phys.hpp"
 #include "dgpu_closure.hpp"
 #include "dgpu_stats.hpp"
 #include "dgpu_courant.hpp"
@@ -117,7 +118,6 @@ struct dgpu_handle {
   void* Aug[MAXA] = {};
   cd* CR[MAXF] = {};
   double* Rp[MAXF] = {};
-  double* CPs = nullptr;
   double* d_dlt = nullptr;  // [2][ny2]: delta_yf, delta_y of the AMD filter width
   double* d_sigma = nullptr;  // filter_chan's horizontal filter, packed [kzr][kxp]
   // les_model_type 6: the network (BF16 forward weights w1t, w2t, w3t; FP32
@@ -184,31 +184,6 @@ int scratch_address(int dev, unsigned char** out) {
   }
   *out = g_scratch_addr[dev];
   return 0;
-}
-
-// Fortran physical array u(0:Nx+1, 0:Nzp+1, 0:Nyp+1) -> compact [j][z][x]
-__global__ void k_pack_phys(const double* __restrict__ fort, double* __restrict__ out, Geo g) {
-  const long long n = (long long)g.ny2 * g.nz * g.nx;
-  for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < n; t += (long long)gridDim.x * blockDim.x) {
-    const int x = (int)(t % g.nx);
-    const long long r = t / g.nx;
-    const int z = (int)(r % g.nz), j = (int)(r / g.nz);
-    out[t] = fort[((long long)j * (g.nz + 2) + z) * (g.nx + 2) + x];
-  }
-}
-
-// packed spectrum [j][k][kxp] -> Fortran cu(0:Nxp, 0:Nz+1, 0:Nyp+1) on the rows
-// k < 2 Nkz + 1, the columns past Nkx zeroed (the host unpack_fourier's map)
-__global__ void k_unpack_four(const cd* __restrict__ comp, cd* __restrict__ fort, Geo g) {
-  const int ldi = g.nx / 2 + 1;
-  const long long n = (long long)g.ny2 * g.kzr * ldi;
-  for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < n; t += (long long)gridDim.x * blockDim.x) {
-    const int i = (int)(t % ldi);
-    const long long r = t / ldi;
-    const int k = (int)(r % g.kzr), j = (int)(r / g.kzr);
-    fort[((long long)j * (g.nz + 2) + k) * ldi + i] =
-        i < g.kxr ? comp[(long long)j * g.pc + (long long)k * g.kxp + i] : cd{0.0, 0.0};
-  }
 }
 
 // filter_chan (for/solver.f90:1597-1685): the horizontal filter of one scalar,
@@ -519,7 +494,10 @@ int launch_inv_z(dgpu_handle* h, int nf, const cd* const* src, void* const* dst,
 }
 
 template <typename T, bool ACC = false>
-int launch_fwd_z(dgpu_handle* h, int nf, void* const* src, cd* const* dst, int j0, int nj) {
+int launch_fwd_z(dgpu_handle* h, int nf, void* const* src, cd* const* dst, int j0, int nj, bool fortran = false) {
+  const long long ldi = h->g.nx / 2 + 1;
+  const long long dj = fortran ? (h->g.nz + 2) * ldi : h->g.pc;
+  const int dk = fortran ? (int)ldi : h->g.kxp, izero = fortran ? (int)ldi : h->g.kxr;
   Ptrs<const cx<T>*, MAXO> s{};
   Ptrs<cd*, MAXO> d{};
   for (int f = 0; f < nf; ++f) { s.p[f] = (const cx<T>*)src[f]; d.p[f] = dst[f]; }
@@ -527,7 +505,7 @@ int launch_fwd_z(dgpu_handle* h, int nf, void* const* src, cd* const* dst, int j
   DG_SWITCH_N(h->g.nz, {
     constexpr int TI = ti_for(N_, sizeof(cx<T>));
     dim3 grid((h->g.kxr + TI - 1) / TI, nj, nf);
-    k_fwd_z<T, N_, TI, 256, ACC><<<grid, 256, 0, h->st>>>(s, d, h->g, j0, tw);
+    k_fwd_z<T, N_, TI, 256, ACC><<<grid, 256, 0, h->st>>>(s, d, h->g, j0, tw, dj, dk, izero);
   });
   HIPCHK(hipGetLastError());
   return 0;
@@ -560,7 +538,11 @@ int launch_inv_x(dgpu_handle* h, int nf, void* const* src, T* const* dst, int j0
 }
 
 template <typename T>
-int launch_fwd_x(dgpu_handle* h, int nf, T* const* src, void* const* dst, int j0, int nj) {
+int launch_fwd_x(dgpu_handle* h, int nf, const T* const* src, void* const* dst, int j0, int nj, bool fortran = false) {
+  // lines of consecutive planes and rows: the device layout [z][j][x], or the
+  // Fortran array u(0:Nx+1, 0:Nzp+1, 0:Nyp+1)
+  const long long sj = fortran ? (long long)(h->g.nz + 2) * (h->g.nx + 2) : h->g.nx;
+  const long long sz = fortran ? h->g.nx + 2 : (long long)h->g.ny2 * h->g.nx;
   Ptrs<const T*, MAXO> s{};
   Ptrs<cx<T>*, MAXO> d{};
   for (int f = 0; f < nf; ++f) { s.p[f] = src[f]; d.p[f] = (cx<T>*)dst[f]; }
@@ -570,10 +552,10 @@ int launch_fwd_x(dgpu_handle* h, int nf, T* const* src, void* const* dst, int j0
     const int pairs = h->g.nz / 2;
     if (pairs % ZP) {
       dim3 grid(pairs, nj, nf);
-      k_fwd_x<T, N_, 1, 256><<<grid, 256, 0, h->st>>>(s, d, h->g, j0, tw);
+      k_fwd_x<T, N_, 1, 256><<<grid, 256, 0, h->st>>>(s, d, h->g, j0, tw, sj, sz);
     } else {
       dim3 grid(pairs / ZP, nj, nf);
-      k_fwd_x<T, N_, ZP, 256><<<grid, 256, 0, h->st>>>(s, d, h->g, j0, tw);
+      k_fwd_x<T, N_, ZP, 256><<<grid, 256, 0, h->st>>>(s, d, h->g, j0, tw, sj, sz);
     }
   });
   HIPCHK(hipGetLastError());
@@ -877,7 +859,7 @@ int ensure_grad_buffers(dgpu_handle* h) {
 
 constexpr int COURANT_BLOCKS = 1024;
 
-// courant's CFL minimum of the physical velocity u1, u2, u3 (FP64 [j][z][x]);
+// courant's CFL minimum of the physical velocity u1, u2, u3 (FP64 [z][j][x]);
 // the block minima stay on the device until dgpu_courant
 int launch_courant(dgpu_handle* h, const double* u1, const double* u2, const double* u3) {
   const dgpu_config& c = h->c;
@@ -1096,7 +1078,7 @@ int substep_les(dgpu_handle* h, int rk, double delta_t, double time, int time_st
   // 7. per-column CN with nu_t / kappa_t (the field systems are independent; the
   //    reference solves the scalars first, for/solver.f90:1004-1007)
   PhysCnArgs<double, T> pa{};
-  pa.g = g; pa.nf = nf; pa.temp2 = temp2; pa.dy = h->d_dy; pa.dyf = h->d_dyf; pa.rowc = h->d_rowc; pa.cp = h->CPs;
+  pa.g = g; pa.nf = nf; pa.temp2 = temp2; pa.dy = h->d_dy; pa.dyf = h->d_dyf; pa.rowc = h->d_rowc;
   for (int e0 = 0; e0 < nf; ++e0) {
     const int e = e0 < NTH ? 3 + e0 : e0 - NTH;  // slot e0 solves field e
     const SolveRows& R = ca.rows[e];
@@ -1116,10 +1098,9 @@ int substep_les(dgpu_handle* h, int rk, double delta_t, double time, int time_st
     pa.tcn[e0] = e < 3 ? temp1 * c.nu_v_scale : temp1 / c.pr[e - 3] * c.nu_v_scale;
   }
   if ((rc = tbeg(h, 8))) return rc;
-  const dim3 pgrid((unsigned)((g.pp + 255) / 256), nf);
   if (inc) {
     PhysCnArgs<float, T> pf{};
-    pf.g = pa.g; pf.nf = pa.nf; pf.temp2 = pa.temp2; pf.dy = pa.dy; pf.dyf = pa.dyf; pf.rowc = pa.rowc; pf.cp = pa.cp;
+    pf.g = pa.g; pf.nf = pa.nf; pf.temp2 = pa.temp2; pf.dy = pa.dy; pf.dyf = pa.dyf; pf.rowc = pa.rowc;
     for (int e0 = 0; e0 < nf; ++e0) {
       pf.field[e0] = pa.field[e0]; pf.blo[e0] = pa.blo[e0]; pf.bhi[e0] = pa.bhi[e0];
       pf.wlo[e0] = pa.wlo[e0]; pf.whi[e0] = pa.whi[e0]; pf.lo_kind[e0] = pa.lo_kind[e0];
@@ -1129,12 +1110,11 @@ int substep_les(dgpu_handle* h, int rk, double delta_t, double time, int time_st
       pf.u[e0] = (float*)h->Pg[3 * pa.field[e0]];
       pf.r[e0] = rinc[pa.field[e0]];
     }
-    k_cn_phys<float, T, true><<<pgrid, 256, 0, h->st>>>(pf);
+    if constexpr (mixed) rc = launch_cn_phys(pf, h->st);
   } else {
-    k_cn_phys<double, T, false><<<pgrid, 256, 0, h->st>>>(pa);
+    rc = launch_cn_phys(pa, h->st);
   }
-  HIPCHK(hipGetLastError());
-  if ((rc = tend(h))) return rc;
+  if (rc || (rc = tend(h))) return rc;
   // courant on the new velocity, before the projection (for/solver.f90:1241-1244)
   if (courant_now)
     if ((rc = launch_courant(h, ucn[0], ucn[1], ucn[2]))) return rc;
@@ -1270,6 +1250,7 @@ int dgpu_create(const dgpu_config* cfg, dgpu_handle** out) {
   g.pc = (long long)g.kxp * g.kzr;
   g.ph = (long long)g.nz * g.kxp;
   g.pp = (long long)g.nz * g.nx;
+  while ((1 << g.lx) < g.nx) ++g.lx;
   auto bail = [&](int code) {
     dgpu_destroy(h);
     return code;
@@ -1308,7 +1289,7 @@ int dgpu_create(const dgpu_config* cfg, dgpu_handle** out) {
   ALLOC(h->d_rowc, sizeof(double) * RC_COUNT * n2);
   if (cfg->use_les) {
     // gradients, eddy viscosity and SGS fields in the transform precision; the
-    // right-hand sides and the solve scratch in FP64
+    // right-hand sides in FP64
     const size_t rbytes = sizeof(double) * g.pp * n2;
     const size_t tbytes = (h->prec == DGPU_MIXED ? sizeof(float) : sizeof(double)) * g.pp * n2;
     for (int f = 0; f < nf; ++f) {
@@ -1320,7 +1301,6 @@ int dgpu_create(const dgpu_config* cfg, dgpu_handle** out) {
     ALLOC(h->NuT, tbytes);
     for (int n = 0; n < h->nth; ++n) ALLOC(h->KapT[n], tbytes);
     for (int m = 0; m < 7 + 2 * h->nth; ++m) ALLOC(h->Aug[m], tbytes);
-    ALLOC(h->CPs, 2 * (size_t)nf * rbytes);
     ALLOC(h->d_dlt, sizeof(double) * 2 * n2);
     if (cfg->les_model_type == 6) {
       ALLOC(h->Cgy, tbytes);
@@ -1498,7 +1478,7 @@ int dgpu_download_les(dgpu_handle* h, double* nu_t, double* kappa_t) {
     std::fill(out, out + fd, 0.0);
     for (int j = 0; j < g.ny2; ++j)
       for (int z = 0; z < g.nz; ++z)
-        std::memcpy(out + ((size_t)j * (g.nz + 2) + z) * (g.nx + 2), &tmp[((size_t)j * g.nz + z) * g.nx],
+        std::memcpy(out + ((size_t)j * (g.nz + 2) + z) * (g.nx + 2), &tmp[pline(g, j, z)],
                     sizeof(double) * g.nx);
   }
   return 0;
@@ -1549,9 +1529,9 @@ int dgpu_closure_counts(dgpu_handle* h, int64_t* network, int64_t* points) {
   HIPCHK(hipMemsetAsync(h->d_ccount, 0, sizeof(c), h->st));
   const Geo& g = h->g;
   if (h->prec == DGPU_MIXED)
-    k_closure_count<float><<<1024, 256, 0, h->st>>>((const float*)h->Cgy, g.pp, g.ny, h->d_ccount);
+    k_closure_count<float><<<1024, 256, 0, h->st>>>((const float*)h->Cgy, g, h->d_ccount);
   else
-    k_closure_count<double><<<1024, 256, 0, h->st>>>((const double*)h->Cgy, g.pp, g.ny, h->d_ccount);
+    k_closure_count<double><<<1024, 256, 0, h->st>>>((const double*)h->Cgy, g, h->d_ccount);
   HIPCHK(hipGetLastError());
   HIPCHK(hipMemcpyAsync(&c, h->d_ccount, sizeof(c), hipMemcpyDeviceToHost, h->st));
   HIPCHK(hipStreamSynchronize(h->st));
@@ -1712,7 +1692,7 @@ int dgpu_courant_physical(dgpu_handle* h, const double* u1, const double* u2, co
   const Geo& g = h->g;
   int rc = ensure_grad_buffers(h);
   if (rc) return rc;
-  // physical Fortran layout u(0:Nx+1, 0:Nzp+1, 0:Nyp+1) -> [j][z][x] in the
+  // physical Fortran layout u(0:Nx+1, 0:Nzp+1, 0:Nyp+1) -> [z][j][x] in the
   // gradient stage's FP64 buffers
   std::vector<double> tmp((size_t)g.pp * g.ny2);
   const double* src[3] = {u1, u2, u3};
@@ -1720,7 +1700,7 @@ int dgpu_courant_physical(dgpu_handle* h, const double* u1, const double* u2, co
   for (int f = 0; f < 3; ++f) {
     for (int j = 0; j < g.ny2; ++j)
       for (int z = 0; z < g.nz; ++z)
-        std::memcpy(&tmp[((size_t)j * g.nz + z) * g.nx], src[f] + ((size_t)j * (g.nz + 2) + z) * (g.nx + 2),
+        std::memcpy(&tmp[pline(g, j, z)], src[f] + ((size_t)j * (g.nz + 2) + z) * (g.nx + 2),
                     sizeof(double) * g.nx);
     HIPCHK(hipMemcpyAsync(dst[f], tmp.data(), tmp.size() * 8, hipMemcpyHostToDevice, h->st));
     HIPCHK(hipStreamSynchronize(h->st));  // tmp is refilled for the next field
@@ -2099,11 +2079,11 @@ int dgpu_fft_xz_to_fourier(dgpu_handle* h, const double* phys, double* four) {
   const Geo& g = h->g;
   int rc = ensure_fft_scratch(h);
   if (rc) return rc;
-  // physical Fortran layout u(0:Nx+1, 0:Nzp+1, 0:Nyp+1) -> [j][z][x]
+  // physical Fortran layout u(0:Nx+1, 0:Nzp+1, 0:Nyp+1) -> [z][j][x]
   std::vector<double> tmp((size_t)g.pp * g.ny2);
   for (int j = 0; j < g.ny2; ++j)
     for (int z = 0; z < g.nz; ++z)
-      std::memcpy(&tmp[((size_t)j * g.nz + z) * g.nx], phys + ((size_t)j * (g.nz + 2) + z) * (g.nx + 2),
+      std::memcpy(&tmp[pline(g, j, z)], phys + ((size_t)j * (g.nz + 2) + z) * (g.nx + 2),
                   sizeof(double) * g.nx);
   HIPCHK(hipMemcpyAsync(h->d_R, tmp.data(), tmp.size() * 8, hipMemcpyHostToDevice, h->st));
   double* rs[1] = {h->d_R};
@@ -2130,7 +2110,7 @@ int dgpu_fft_xz_to_physical(dgpu_handle* h, const double* four, double* phys) {
   HIPCHK(hipStreamSynchronize(h->st));
   for (int j = 0; j < g.ny2; ++j)
     for (int z = 0; z < g.nz; ++z)
-      std::memcpy(phys + ((size_t)j * (g.nz + 2) + z) * (g.nx + 2), &tmp[((size_t)j * g.nz + z) * g.nx],
+      std::memcpy(phys + ((size_t)j * (g.nz + 2) + z) * (g.nx + 2), &tmp[pline(g, j, z)],
                   sizeof(double) * g.nx);
   return 0;
 }
@@ -2148,20 +2128,15 @@ int dgpu_fft_xz_to_fourier_noalloc(dgpu_handle* h, const double* phys, double* f
     return fail(2, "dgpu_fft_xz_to_fourier_noalloc: this grid needs " + std::to_string(rb + hb + cb) +
                        " bytes of transform scratch; the allocation-free entry point holds " +
                        std::to_string(kNoallocScratchBytes));
-  double* R = (double*)h->noalloc;
-  cd* H = (cd*)(h->noalloc + rb);
-  cd* C = (cd*)(h->noalloc + rb + hb);
-  const int nb = 1024;
-  k_pack_phys<<<nb, 256, 0, h->st>>>(phys, R, g);
-  HIPCHK(hipGetLastError());
-  double* rs[1] = {R};
-  void* hs[1] = {H};
-  cd* cs[1] = {C};
+  // the transforms read and write the Fortran arrays themselves (the scratch bound
+  // above is the interface's); the x-spectra are complete before four is written,
+  // so the two may alias
+  const double* rs[1] = {phys};
+  void* hs[1] = {h->noalloc + rb};
+  cd* cs[1] = {(cd*)four};
   int rc;
-  if ((rc = launch_fwd_x<double>(h, 1, rs, hs, 0, g.ny2))) return rc;
-  if ((rc = launch_fwd_z<double>(h, 1, hs, cs, 0, g.ny2))) return rc;
-  k_unpack_four<<<nb, 256, 0, h->st>>>(C, (cd*)four, g);
-  HIPCHK(hipGetLastError());
+  if ((rc = launch_fwd_x<double>(h, 1, rs, hs, 0, g.ny2, true))) return rc;
+  if ((rc = launch_fwd_z<double>(h, 1, hs, cs, 0, g.ny2, true))) return rc;
   HIPCHK(hipStreamSynchronize(h->st));
   return 0;
 }
