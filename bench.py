@@ -49,8 +49,6 @@ def kernel_bytes(cfg, mixed):
         # DNS x pass marching in y: the x-spectra of planes jlo-1..ny+1 in, the
         # product spectra of planes jlo..ny out (physical fields stay on chip)
         "k_xmarch": nf * cfg.kxr * cfg.nz * 2 * s * (nj + 2) + no * Hj,
-        # LES x pass: physical fields (and SGS fields) in, product spectra out
-        "k_xprod": nf * Rtj + no * Hj,
         "k_fwdz_nl": no * Hj + nf * Cj_t,
         # nonlinear terms, state, cp and (rk 2, 3: 2 of 3 launches) old cf in; cf and state out
         "k_cn": nf * Cj_t + (nf + 1) * C + (2.0 / 3.0) * nf * Cj + nf * Cj + nf * C,
@@ -59,21 +57,19 @@ def kernel_bytes(cfg, mixed):
     # DNS: the same with the projection in the kernel: the pressure goes out too
     out["k_column"] = out["k_cn"] + C
     if cfg.use_les:
-        # physical fields: R8 FP64, Rt in the transform precision; na SGS addition fields
+        # physical fields: R8 FP64, Rt in the transform precision
         R8 = cfg.nx * cfg.nz * 8 * ny2
         Hf = cfg.kxr * cfg.nz * 2 * 4 * ny2        # float x-spectrum (increment transforms)
         Rf = cfg.nx * cfg.nz * 4 * ny2
-        na = 7 + 2 * cfg.n_th
         learned = cfg.les_model_type == 6
         out["k_bc_post"] = nf * 6 * C / ny2
         # z inverse of v and dv/dz (2 nf), x inverse of v, dv/dx, dv/dz (3 nf)
         out["les_grad"] = 2 * nf * C + 2 * nf * H + 3 * nf * H + 3 * nf * Rt
-        # gradient fields in; nu_t, kappa_t, SGS fields out (the learned model also
-        # reads its four coefficient planes)
-        out["k_amd"] = 3 * nf * Rt + (1 + cfg.n_th + na) * Rt + (4 * Rt if learned else 0)
+        # LES x pass: gradient fields in; nu_t, kappa_t and the product spectra out (the
+        # learned model also reads its four coefficient planes)
+        out["k_les_products"] = 3 * nf * Rt + (1 + cfg.n_th) * Rtj + no * Hj + (4 * Rt if learned else 0)
         if learned:
             out["k_closure"] = 3 * nf * Rt + 4 * Rt
-        out["k_xprod"] += na * Rtj
         # assembly only: the right-hand side goes out instead of the solve
         out["k_cn"] = nf * Cj_t + (nf + 1) * C + (2.0 / 3.0) * nf * Cj + nf * Cj + nf * C
         npts = cfg.nx * cfg.nz * ny2

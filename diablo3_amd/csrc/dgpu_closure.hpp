@@ -9,8 +9,8 @@
 // scalar gradient of amd_th_gy; each wave stages its 64 points in LDS and
 // evaluates them as 4 MFMA tiles of 16 samples.  It writes the velocity and
 // scalar coefficients at GY (1/time; nu_t = C^2 D2 coefficient) with the sign
-// bit marking a fallback point (the AMD value, stored negated).  k_amd<..., 6>
-// takes |coefficient| at GY, and at GYF j the mean of GY j and j+1 when both
+// bit marking a fallback point (the AMD value, stored negated).  k_les_products
+// (model 6) takes |coefficient| at GY, and at GYF j the mean of GY j and j+1 when both
 // are network points, else the type-5 GYF coefficient, so that a handle with
 // no network (or an empty envelope) steps exactly as type 5.
 // Feature mode (dgpu_les_features) evaluates the features at the GYF points of
@@ -134,7 +134,9 @@ __global__ __launch_bounds__(256) void k_closure(ClosureArgs c) {
   const bool live = q0 < g.pp;
   const long long qf = live ? q0 : g.pp - 1, q = pcol(g, qf);  // every lane takes part in the MFMA tiles
   const int ny = g.ny;
+  T win[3 * (3 + NTH)][4];
   AmdIn<T> in;
+  in.w = win;
   load_window<T, 3 * (3 + NTH)>(in, a, j, q);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   // step mode: GY rows 2..Nyp; feature mode: GYF rows jf0..Nyp-1
@@ -142,7 +144,7 @@ __global__ __launch_bounds__(256) void k_closure(ClosureArgs c) {
   float fe[MLP_INP];
 #pragma unroll
   for (int k = 0; k < MLP_INP; ++k) fe[k] = 0.f;
-  // the AMD values in the transform precision T (as k_amd's type 5), the features in float
+  // the AMD values in the transform precision T (as the model's type 5), the features in float
   T amd_v = T(0), amd_t = T(0);
   float s2 = 0.f;
   if (on) {

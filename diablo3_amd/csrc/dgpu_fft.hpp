@@ -307,8 +307,7 @@ __device__ __forceinline__ void fft_lds_wave(cx<T>* __restrict__ s, int ld,
 // fft_lds_wave and one barrier where every wave has a line (LINES >= NT / 64)
 // and a line fills a wave (N >= 64), else fft_lds: either way the lines are
 // complete for every thread on return.  Above N = 256 only in FP64 (measured at
-// 512x257x512: FP64 k_xprod 3.27 -> 3.12 ms and k_fwdz_nl 1.04 -> 0.91 ms, but
-// float k_xprod 1.37 -> 1.41 and k_fwdz_nl 0.73 -> 0.82).
+// 512x257x512: FP64 k_fwdz_nl 1.04 -> 0.91 ms, but float 0.73 -> 0.82).
 template <typename T, int N, int LINES, int NT, int DIR>
 __device__ __forceinline__ void fft_lds_sync(cx<T>* __restrict__ s, int ld,
                                              const cx<T>* __restrict__ tw, int tid) {

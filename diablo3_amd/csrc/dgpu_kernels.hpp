@@ -68,23 +68,40 @@ __device__ __forceinline__ int xcd_tile(int b, int total, int K) {
 }
 constexpr int XCD_K = 16;
 
+// Blocks of a batch of nf fields over ns places: XCD x (blocks x, x + 8, ...) takes
+// runs of K consecutive places through all fields before its next run, so that
+// fields with a common source (v and dv/dz) find it in its L2 (512x257x512 FP64, 8
+// fields of 4 sources: 1234 -> 1066 us).  batch_grid
+// blocks in all; false for those past the last place.
+__host__ __device__ __forceinline__ int batch_grid(int ns, int nf, int K) { return (ns + 8 * K - 1) / (8 * K) * 8 * K * nf; }
+__device__ __forceinline__ bool batch_place(int b, int ns, int nf, int K, int& place, int& f) {
+  const int t = b >> 3, r = t / K;
+  f = r % nf;
+  place = (r / nf * 8 + (b & 7)) * K + t % K;
+  return place < ns;
+}
+
 // ---------------------------------------------------------------------------
 // z transforms: inverse (packed C -> H) and forward (H -> packed C)
 // ---------------------------------------------------------------------------
+// Places of a run on one XCD: neighbouring column tiles where a tile's rows are less
+// than a 128-byte line (each line is then read by two of them), else one.
+template <typename T, int TI>
+constexpr int ZK = TI * sizeof(cx<T>) < 128 ? XCD_K : 1;
 // Field f of a batch with bit f of dzmask set is multiplied by i kz before the
 // transform (the x-spectrum of its z derivative).
 template <typename T, int NZ, int TI, int NT>
 __global__ __launch_bounds__(NT) void k_inv_z(Ptrs<const cd*, MAXO> src, Ptrs<cx<T>*, MAXO> dst,
-                                              Geo g, int j0, const cx<T>* __restrict__ tw,
+                                              Geo g, int j0, int nj, int nf, const cx<T>* __restrict__ tw,
                                               const double* __restrict__ kz, unsigned dzmask) {
   constexpr int LD = NZ + 1;
+  const int nib = (g.kxr + TI - 1) / TI;
+  int tt, f;
+  if (!batch_place(blockIdx.x, nib * nj, nf, ZK<T, TI>, tt, f)) return;
   __shared__ cx<T> s[TI * LD];
   __shared__ cx<T> stw[NZ];  // twiddles
   stage_twiddles<T, NZ, NT>(stw, tw, threadIdx.x);
-  // grid (column blocks, planes, fields), taken in xcd_tile order
-  const int nib = gridDim.x, nj = gridDim.y;
-  const int tt = xcd_tile(blockIdx.x + nib * (blockIdx.y + nj * blockIdx.z), nib * nj * gridDim.z, XCD_K);
-  const int f = tt / (nib * nj), j = j0 + (tt / nib) % nj, i0 = (tt % nib) * TI, tid = threadIdx.x;
+  const int j = j0 + tt / nib, i0 = (tt % nib) * TI, tid = threadIdx.x;
   const cd* __restrict__ C = src.p[f] + (long long)j * g.pc;
   const bool dz = (dzmask >> f) & 1u;
   // every load of the thread first, then the LDS stores (the loads overlap)
@@ -157,24 +174,6 @@ __global__ __launch_bounds__(NT) void k_fwd_z(Ptrs<const cx<T>*, MAXO> src, Ptrs
 // ---------------------------------------------------------------------------
 // x transforms, two real lines (z, z+1) per complex transform
 // ---------------------------------------------------------------------------
-// Hermitian completion of the pair of half spectra A (line z), B (line z+1) into
-// the length-NX spectrum of A + iB; bins i > Nkx are zero and the imaginary part
-// of each DC bin is dropped (a real line's DC bin is real; FFTW's c2r ignores it).
-template <typename T>
-__device__ __forceinline__ cx<T> pair_spectrum(const cx<T>* __restrict__ A,
-                                               const cx<T>* __restrict__ B, int n, int nx, int nkx) {
-  if (n == 0) return {A[0].x, B[0].x};
-  if (n <= nkx) {
-    cx<T> a = A[n], b = B[n];
-    return {a.x - b.y, a.y + b.x};
-  }
-  if (n >= nx - nkx) {
-    cx<T> a = A[nx - n], b = B[nx - n];
-    return {a.x + b.y, b.x - a.y};
-  }
-  return {T(0), T(0)};
-}
-
 // split the spectrum Z of a + i b into the half spectra of a and b at bin i
 template <typename T>
 __device__ __forceinline__ void pair_split(const cx<T>* __restrict__ Zl, int i, int nx, cx<T>& A, cx<T>& B) {
@@ -197,9 +196,11 @@ __global__ __launch_bounds__(NT) void k_inv_x(Ptrs<const cx<T>*, MAXO> src, Ptrs
   const cx<T>* __restrict__ H = src.p[f] + (long long)j * g.ph;
   const bool dx = (dxmask >> f) & 1u;
   // Each half-spectrum bin m = 0..NX/2 of the two lines is loaded once and gives
-  // both bins m and NX - m of the pair spectrum (pair_spectrum written out for the
-  // two halves; for an x derivative the bins times i kx, DC zero); every load of
-  // the thread first, then the LDS stores (the loads overlap).
+  // both bins m and NX - m of the pair spectrum (the hermitian completion of A + iB
+  // written out for the two halves; for an x derivative the bins times i kx, DC zero);
+  // bins i > Nkx are zero, and the imaginary part of each DC bin is dropped (a real
+  // line's DC bin is real; FFTW's c2r ignores it).  Every load of the thread first,
+  // then the LDS stores (the loads overlap).
   constexpr int HB = NX / 2 + 1;
   constexpr int PER = (ZP * HB + NT - 1) / NT;
   cx<T> lo[PER], hi[PER];
@@ -319,13 +320,6 @@ struct XProdArgs {
   const void* hin[MAXF];   // x-spectra of u1, u2, u3, th_n (all planes)
   void* hout[MAXO];        // N1, N2, N3, Z1, Z2, Z3, (Nt, Zt) per scalar
   const void* tw;
-  // LES: physical SGS fields added to products 1, 0, 2, 5, 6, 3, 4, (8, 9) + 3n
-  // (tau_11, tau_13, tau_33, the two stress fluxes, the two GY stresses, the
-  // scalar fluxes); null for DNS
-  const void* aug[7 + 2 * MAXTH];
-  // the fields in physical space ([z][j][x], T), all planes, written by the
-  // inverse x transform; the kernel reads the three planes of its x columns
-  const void* phys[MAXF];
 };
 
 // The NP = 8 + 3 NTH product lines of one column x at plane j, from the physical
@@ -437,68 +431,6 @@ __device__ __forceinline__ void xprod_store(const cx<T>* __restrict__ s, const G
     H[(long long)z * g.kxp + i] = v2{rnx * ra.x, rnx * ra.y};
     H[(long long)(z + 1) * g.kxp + i] = v2{rnx * rb.x, rnx * rb.y};
   }
-}
-
-// A separate inverse x transform has written the physical fields once per
-// plane; each block reads the three planes j-1..j+1 of its line pair (z, z+1),
-// forms the products and forward-transforms them in LDS.  (The LES x pass: the
-// physical fields exist anyway for the closure, and the SGS fields are added to
-// the products.)
-template <typename T, int NX, int NT, int NTH, bool LES>
-__global__ __launch_bounds__(NT) void k_xprod(XProdArgs a) {
-  constexpr int NP = 8 + 3 * NTH;
-  __shared__ cx<T> s[NP * NX];
-  __shared__ cx<T> stw[NX];  // twiddles
-  stage_twiddles<T, NX, NT>(stw, (const cx<T>*)a.tw, threadIdx.x);
-  const Geo& g = a.g;
-  const int tid = threadIdx.x, z = 2 * blockIdx.x, j = a.jlo + blockIdx.y;
-  __syncthreads();  // the twiddle table
-  // (field f, plane j-1+d) of the line pair (z, z+1) at column x
-  auto field = [&](int f, int d, int x) -> cx<T> {
-    const T* R = (const T*)a.phys[f] + pline(g, j - 1 + d, z) + x;
-    return cx<T>{R[0], R[(long long)g.ny2 * NX]};
-  };
-  for (int x = tid; x < NX; x += NT) {
-    cx<T> U1[3], U2[3], U3[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      U1[d] = field(0, d, x);
-      U2[d] = field(1, d, x);
-      U3[d] = field(2, d, x);
-    }
-    cx<T> TH[NTH > 0 ? NTH : 1][3];
-#pragma unroll
-    for (int n = 0; n < NTH; ++n)
-#pragma unroll
-      for (int d = 0; d < 3; ++d) TH[n][d] = field(3 + n, d, x);
-    cx<T> P[NP];
-    xprod_products<T, NTH>(a, j, U1, U2, U3, TH, P);
-    if constexpr (LES) {
-      const long long pz = pline(g, j, z) + x;
-      auto A = [&](int m) {
-        const T* p = (const T*)a.aug[m];
-        return cx<T>{p[pz], p[pz + (long long)g.ny2 * NX]};
-      };
-      P[1] = P[1] + A(0);
-      P[0] = P[0] + A(1);
-      P[2] = P[2] + A(2);
-      P[5] = P[5] + A(3);
-      P[6] = P[6] + A(4);
-      P[3] = P[3] + A(5);
-      P[4] = P[4] + A(6);
-#pragma unroll
-      for (int n = 0; n < NTH; ++n) {
-        P[8 + 3 * n] = P[8 + 3 * n] + A(7 + 2 * n);
-        P[9 + 3 * n] = P[9 + 3 * n] + A(8 + 2 * n);
-      }
-    }
-    // each thread writes only column x of the product lines
-#pragma unroll
-    for (int p = 0; p < NP; ++p) s[p * NX + swz<T>(x)] = P[p];
-  }
-  __syncthreads();
-  fft_lds_sync<T, NX, NP, NT, -1>(s, NX, stw, tid);
-  xprod_store<T, NX, NT, NTH>(s, g, a.hout, a.kx, z, j, tid);
 }
 
 // The DNS x pass in one kernel, marching in y.  Block (z pair, segment) owns the

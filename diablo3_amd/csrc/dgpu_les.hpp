@@ -11,10 +11,11 @@
 //    per transported variable instead of 27 transforms (every strain, rotation
 //    and invariant tensor entry is a pointwise combination of these, and
 //    d/dy is the reference's own difference stencil applied in physical space);
-//  * k_amd evaluates nu_t, kappa_t and the SGS stresses per point and writes them
-//    as additions to the nonlinear product fields whose spectral derivatives the
+//  * k_les_products evaluates nu_t, kappa_t and the SGS stresses per point and adds
+//    the stresses to the nonlinear products whose spectral derivatives the
 //    reference applies to the stress (tau_11 joins u1u1, tau_13 joins u1u3, ...),
-//    so the stress divergence rides on the product transforms of k_xprod;
+//    so the stress divergence rides on the products' x transforms, which follow in
+//    the same kernel;
 //  * the Crank–Nicolson solve with nu_t runs per physical (x, z) column
 //    (k_cn_phys), as in the reference, since nu_t varies in x and z.
 // Transforms are linear, so moving a linear operation across one changes only
@@ -24,7 +25,6 @@
 
 namespace dgpu {
 
-constexpr int MAXA = 7 + 2 * MAXTH;  // SGS addition fields
 constexpr double C_AMD = 0.2887;     // for/les.f90:25
 constexpr double C_SMAG = 0.17;      // for/les.f90:24
 constexpr double BETA_SGS = 3.0;     // for/les.f90:43
@@ -119,9 +119,10 @@ __global__ __launch_bounds__(256) void k_bc_post(BcArgs a) {
 // ---------------------------------------------------------------------------
 // AMD model per point (for/les.f90:571-797, 1213-1346).
 // Inputs (physical, [z][j][x], all planes): for each transported field v in
-// (u1, u2, u3, th_n): v, dv/dx, dv/dz.  Outputs, on every plane (zero where the
-// reference adds nothing):
-//   nu_t, kappa_t_n            at GY points, zero at j = 0, 1, 2, Nyp, Nyp+1
+// (u1, u2, u3, th_n): v, dv/dx, dv/dz.  Outputs (zero where the reference adds
+// nothing):
+//   nu_t, kappa_t_n            at GY points, zero at j = 0, 1, 2, Nyp, Nyp+1 (written on
+//                              the planes the products have; zero from the start on the others)
 //   A0 = tau_11  (joins u1u1)       A1 = tau_13 (joins u1u3)   rows jstart..Nyp-1
 //   A2 = tau_33  (joins u3u3)       A3 = (tau_12(j+1)-tau_12(j))/dyf(j)  (u1 flux)
 //   A4 = (tau_23(j+1)-tau_23(j))/dyf(j)  (u3 flux)                        rows jstart..Nyp-1
@@ -141,7 +142,6 @@ struct AmdArgs {
   const void* f[3 * MAXF];              // v, dv/dx, dv/dz per transported field
   void* nut;
   void* kap[MAXTH];
-  void* aug[MAXA];
   // les_model_type 6: the learned closure's coefficients at GY (k_closure), in
   // the transform precision T, sign bit set where the point took the AMD value
   const void* cgy;   // velocity
@@ -165,7 +165,7 @@ struct Gy {
 // at() is called with rows j + const, so the window index folds to a constant.
 template <typename T>
 struct AmdIn {
-  T w[3 * MAXF][4];
+  T (*w)[4];       // the kernel's array (apart from j0, so that it can be split into registers)
   int j0;          // j - 1
   int nx;          // from row to row
   __device__ T at(int f, int row, long long) const { return w[f][row - j0]; }
@@ -416,11 +416,14 @@ template <int MODEL, typename T>
 __device__ __forceinline__ T tau_gy(const AmdIn<T>& in, const AmdArgs& a, int e, int j, long long q, T coef) {
   using R = T;
   const R dlt = R(a.dlt[a.g.ny2 + j]);
-  if (MODEL != 1 && j == 1) {
-    const R dvdy = (in.at(e ? 6 : 0, 1, q) - in.at(e ? 6 : 0, 0, q)) * R(rq(a, 1)[RC_RDY]);
-    return dlt * R(0.5) * (dvdy + in.at(e ? 5 : 4, 1, q));
-  }
-  return dlt * (coef * (R(0.5) * in.at(e ? 5 : 4, j, q)));
+  const R half = R(0.5) * in.at(e ? 5 : 4, j, q);
+  if constexpr (MODEL == 1) return dlt * (coef * half);
+  // the row asked for through a copy of j: where the compiler knows that j is 1 it
+  // addresses the window by 2 - j, in memory
+  int jc = j;
+  asm("" : "+s"(jc));
+  const R dvdy = (in.at(e ? 6 : 0, j, q) - in.at(e ? 6 : 0, j - 1, q)) * R(rq(a, j)[RC_RDY]);
+  return jc == 1 ? dlt * R(0.5) * (dvdy + in.at(e ? 5 : 4, j, q)) : dlt * (coef * half);
 }
 
 // Block b of a 1D grid over (256-point block qb, row j) pairs.  The dispatcher
@@ -439,20 +442,18 @@ __device__ __forceinline__ void xcd_rows(int b, int nqb, int nj, int& qb, int& j
   qb = (t / nj) * 8 + (b & 7);
 }
 
+// The model at one point of row j: nu_t and kappa_t (GY), and the additions to the
+// products.
+template <typename T, int NTH>
+struct AmdOut {
+  T nut, kap[NTH > 0 ? NTH : 1], A[7 + 2 * NTH];
+};
 template <typename T, int NTH, int MODEL>
-__global__ __launch_bounds__(256) void k_amd(AmdArgs a) {
+__device__ __forceinline__ void amd_point(const AmdIn<T>& in, const AmdArgs& a, int j, long long q, AmdOut<T, NTH>& r) {
   using R = T;
   const Geo& g = a.g;
-  int qb, j;
-  xcd_rows(blockIdx.x, (int)((g.pp + 255) / 256), g.ny2, qb, j);
-  const long long q0 = (long long)qb * 256 + threadIdx.x;
-  if (q0 >= g.pp) return;
-  const long long q = pcol(g, q0);
-  AmdIn<T> in;
-  load_window<T, 3 * (3 + NTH)>(in, a, j, q);
   const int ny = g.ny;
   const long long o = (long long)j * g.nx + q;
-  auto put = [&](void* p, R v) { ((T*)p)[o] = (T)v; };
   // the model coefficient at GY j and j + 1, each evaluated once: nu_t, the two
   // stresses at GY j and the GYF flux differences take them (row 1 of types 4
   // and 5 needs none)
@@ -461,71 +462,228 @@ __global__ __launch_bounds__(256) void k_amd(AmdArgs a) {
   const R cj1 = (j >= a.jstart && j <= ny - 1) ? model_gy<MODEL>(in, a, j + 1, q) : R(0.0);
   const double* rc = rq(a, j);
   // nu_t at GY j (zero on the wall rows of ghost_les_mpi)
-  R nut = R(0.0);
-  if (j >= 3 && j <= ny - 1) nut = -R(0.5) * R(a.dlt[g.ny2 + j]) * cj;
-  put(a.nut, nut);
+  r.nut = R(0.0);
+  if (j >= 3 && j <= ny - 1) r.nut = -R(0.5) * R(a.dlt[g.ny2 + j]) * cj;
+#pragma unroll
+  for (int m = 0; m < 7 + 2 * NTH; ++m) r.A[m] = R(0.0);
   // GYF stresses, rows j1..j2 = jstart..Nyp-1
-  R A0 = R(0.0), A1 = R(0.0), A2 = R(0.0), A3 = R(0.0), A4 = R(0.0);
   if (j >= a.jstart && j <= ny - 1) {
     const R dyf = R(a.dlt[j]) * model_gyf<MODEL>(in, a, j, q);
     const R du1dz = in.at(2, j, q), du3dx = in.at(7, j, q);
-    A0 = dyf * in.at(1, j, q);
-    A1 = dyf * (R(0.5) * (du1dz + du3dx));
-    A2 = dyf * in.at(8, j, q);
+    r.A[0] = dyf * in.at(1, j, q);
+    r.A[1] = dyf * (R(0.5) * (du1dz + du3dx));
+    r.A[2] = dyf * in.at(8, j, q);
     const R rdyf = R(rc[RC_RDYF]);
-    A3 = (tau_gy<MODEL>(in, a, 0, j + 1, q, cj1) - tau_gy<MODEL>(in, a, 0, j, q, cj)) * rdyf;
-    A4 = (tau_gy<MODEL>(in, a, 1, j + 1, q, cj1) - tau_gy<MODEL>(in, a, 1, j, q, cj)) * rdyf;
+    r.A[3] = (tau_gy<MODEL>(in, a, 0, j + 1, q, cj1) - tau_gy<MODEL>(in, a, 0, j, q, cj)) * rdyf;
+    r.A[4] = (tau_gy<MODEL>(in, a, 1, j + 1, q, cj1) - tau_gy<MODEL>(in, a, 1, j, q, cj)) * rdyf;
   }
-  put(a.aug[0], A0); put(a.aug[1], A1); put(a.aug[2], A2); put(a.aug[3], A3); put(a.aug[4], A4);
   // GY stresses and the explicit cross terms, rows 2..Nyp
-  R A5 = R(0.0), A6 = R(0.0);
   if (j >= 2 && j <= ny) {
     const R rdy = R(rc[RC_RDY]);
-    A5 = tau_gy<MODEL>(in, a, 0, j, q, cj) - nut * ((in.at(0, j, q) - in.at(0, j - 1, q)) * rdy);
-    A6 = tau_gy<MODEL>(in, a, 1, j, q, cj) - nut * ((in.at(6, j, q) - in.at(6, j - 1, q)) * rdy);
+    r.A[5] = tau_gy<MODEL>(in, a, 0, j, q, cj) - r.nut * ((in.at(0, j, q) - in.at(0, j - 1, q)) * rdy);
+    r.A[6] = tau_gy<MODEL>(in, a, 1, j, q, cj) - r.nut * ((in.at(6, j, q) - in.at(6, j - 1, q)) * rdy);
   }
-  put(a.aug[5], A5); put(a.aug[6], A6);
-  if constexpr (MODEL == 1 || MODEL == 4) {
-    // les_chan_th types 1 and 4 (for/les.f90:1118-1193): kappa_t = nu_t (GY), and
-    // cfth += ikx F(kappa_t dth/dx) + ikz F(kappa_t dth/dz) on rows jstart_th..jend_th
-#pragma unroll
-    for (int n = 0; n < NTH; ++n) {
-      const int ft = 3 * (3 + n);
-      put(a.kap[n], nut);
-      const bool row = (j >= a.jstart_th[n] && j <= a.jend_th[n]);
-      put(a.aug[7 + 2 * n], row ? -(nut * in.at(ft + 1, j, q)) : R(0.0));
-      put(a.aug[8 + 2 * n], row ? -(nut * in.at(ft + 2, j, q)) : R(0.0));
-    }
-    return;
-  }
-  // scalars (les_chan_th type 5; type 6 reads the learned coefficients)
 #pragma unroll
   for (int n = 0; n < NTH; ++n) {
     const int ft = 3 * (3 + n);
-    R kap = R(0.0), fx = R(0.0), fz = R(0.0);
-    // kappa_t at GY j (for/les.f90:1259-1306, 1344-1348)
-    if (j >= 3 && j <= ny - 1) {
-      R c;
-      if constexpr (MODEL == 6) c = fabs((R)((const T*)a.kgy)[o]);
-      else c = amd_th_gy(in, a, ft, j, q).c;
-      kap = -R(0.5) * R(a.dlt[g.ny2 + j]) * c;
-    }
-    put(a.kap[n], kap);
-    // SGS flux at GYF j (for/les.f90:1221-1256, 1310-1318, 1372-1393)
-    if (j >= a.jstart_th[n] && j <= a.jend_th[n]) {
-      R s1;
-      if constexpr (MODEL == 6) {
-        const R k0 = (R)((const T*)a.kgy)[o], k1 = (R)((const T*)a.kgy)[o + g.nx];
-        s1 = (!signbit(k0) && !signbit(k1)) ? R(0.5) * (k0 + k1) : amd_th_gyf(in, a, ft, j, q).c;
-      } else {
-        s1 = amd_th_gyf(in, a, ft, j, q).c;
+    const bool row = (j >= a.jstart_th[n] && j <= a.jend_th[n]);
+    r.kap[n] = R(0.0);
+    if constexpr (MODEL == 1 || MODEL == 4) {
+      // les_chan_th types 1 and 4 (for/les.f90:1118-1193): kappa_t = nu_t (GY), and
+      // cfth += ikx F(kappa_t dth/dx) + ikz F(kappa_t dth/dz) on rows jstart_th..jend_th
+      r.kap[n] = r.nut;
+      r.A[7 + 2 * n] = row ? -(r.nut * in.at(ft + 1, j, q)) : R(0.0);
+      r.A[8 + 2 * n] = row ? -(r.nut * in.at(ft + 2, j, q)) : R(0.0);
+    } else {
+      // les_chan_th type 5; type 6 reads the learned coefficients.
+      // kappa_t at GY j (for/les.f90:1259-1306, 1344-1348)
+      if (j >= 3 && j <= ny - 1) {
+        R c;
+        if constexpr (MODEL == 6) c = fabs((R)((const T*)a.kgy)[o]);
+        else c = amd_th_gy(in, a, ft, j, q).c;
+        r.kap[n] = -R(0.5) * R(a.dlt[g.ny2 + j]) * c;
       }
-      const R f = R(0.5) * R(a.dlt[j]) * s1;
-      fx = f * in.at(ft + 1, j, q);
-      fz = f * in.at(ft + 2, j, q);
+      // SGS flux at GYF j (for/les.f90:1221-1256, 1310-1318, 1372-1393)
+      if (row) {
+        R s1;
+        if constexpr (MODEL == 6) {
+          const R k0 = (R)((const T*)a.kgy)[o], k1 = (R)((const T*)a.kgy)[o + g.nx];
+          s1 = (!signbit(k0) && !signbit(k1)) ? R(0.5) * (k0 + k1) : amd_th_gyf(in, a, ft, j, q).c;
+        } else {
+          s1 = amd_th_gyf(in, a, ft, j, q).c;
+        }
+        const R f = R(0.5) * R(a.dlt[j]) * s1;
+        r.A[7 + 2 * n] = f * in.at(ft + 1, j, q);
+        r.A[8 + 2 * n] = f * in.at(ft + 2, j, q);
+      }
     }
-    put(a.aug[7 + 2 * n], fx);
-    put(a.aug[8 + 2 * n], fz);
+  }
+}
+
+// The products of xprod_products at one point, plus the SGS additions.
+template <typename T, int NTH>
+__device__ __forceinline__ void les_products(const XProdArgs& x, const AmdIn<T>& in, int j, const AmdOut<T, NTH>& r,
+                                             T* P) {
+  const int ny = x.g.ny;
+  // rows j-1, j, j+1 of u1, u2, u3
+  const T u0 = in.w[0][0], u = in.w[0][1], up = in.w[0][2];
+  const T v0 = in.w[3][0], v = in.w[3][1], vp = in.w[3][2];
+  const T w0 = in.w[6][0], w = in.w[6][1], wp = in.w[6][2];
+  const double* rc = x.rowc + (long long)j * RC_COUNT;
+  const T rdy = (T)rc[RC_RDY], r2f = T(0.5) * (T)rc[RC_RDYF];
+  const T dyfj = (T)x.dyf[j], dyfm = (T)x.dyf[j - 1];
+  const T cint = T(0.5) * rdy;
+#pragma unroll
+  for (int p = 0; p < 8 + 3 * NTH; ++p) P[p] = T(0);
+  if (j >= x.jstart && j <= x.jend) {
+    P[0] = w * u + r.A[1];
+    P[1] = u * u + r.A[0];
+    P[2] = w * w + r.A[2];
+    P[5] = (up * vp + u * vp - u * v - u0 * v) * r2f + r.A[3];
+    P[6] = (wp * vp + w * vp - w * v - w0 * v) * r2f + r.A[4];
+  }
+  if (j >= 2 && j <= ny) {
+    P[3] = ((dyfj * u + dyfm * u0) * cint) * v + r.A[5];
+    P[4] = ((dyfj * w + dyfm * w0) * cint) * v + r.A[6];
+    const T ap = v + vp, am = v + v0;
+    P[7] = (T(0.25) * (ap * ap) - T(0.25) * (am * am)) * rdy;
+  }
+#pragma unroll
+  for (int n = 0; n < NTH; ++n) {
+    const T t0 = in.w[9 + 3 * n][0], t = in.w[9 + 3 * n][1], tp = in.w[9 + 3 * n][2];
+    if (j >= x.jstart_th[n] && j <= x.jend_th[n]) {
+      P[8 + 3 * n] = t * u + r.A[7 + 2 * n];
+      P[9 + 3 * n] = t * w + r.A[8 + 2 * n];
+      P[10 + 3 * n] = (tp * vp + t * vp - t * v - t0 * v) * r2f;
+    }
+  }
+}
+
+// SPLIT: the order of the product lines, u1's and u3's equations (u1u1, flux of u1,
+// u3u1, flux of u3, u3u3), then u2's and the scalars' (u1u2i, flux, u3u2i; th u1,
+// flux, th u3).
+template <int NTH>
+constexpr int les_line(int p) {
+  constexpr int first[8] = {1, 5, 0, 6, 2, 3, 7, 4};
+  if (p < 8) return first[p];
+  const int n = (p - 8) / 3, r = (p - 8) % 3;
+  return 8 + 3 * n + (r == 0 ? 0 : (r == 1 ? 2 : 1));
+}
+// xprod_store for the lines of one half.
+template <typename T, int NX, int NT, int NTH, int HALF>
+__device__ __forceinline__ void les_store(const cx<T>* __restrict__ s, const Geo& g, void* const* hout,
+                                          const double* __restrict__ kxt, int z, int j, int tid) {
+  constexpr int NO = HALF == 0 ? 4 : 2 + 2 * NTH;
+  const T rnx = T(1) / T(NX);
+#pragma unroll
+  for (int t = 0; t < NO; ++t) {
+    // output, derivative line (times -ikx) and flux line of the half; no flux: a copy
+    const int o = HALF == 0 ? (t == 0 ? 0 : t == 1 ? 2 : t == 2 ? 3 : 5) : (t == 0 ? 1 : t == 1 ? 4 : 4 + t);
+    const int pd = HALF == 0 ? (t == 0 ? 0 : t == 3 ? 4 : 2) : (t < 2 ? 2 * t : 3 + 3 * ((t - 2) / 2) + 2 * (t % 2));
+    const int pf = HALF == 0 ? (t == 0 ? 1 : t == 1 ? 3 : -1)
+                             : (t == 0 ? 1 : t == 1 || t % 2 == 1 ? -1 : 4 + 3 * ((t - 2) / 2));
+    cx<T>* H = (cx<T>*)hout[o] + (long long)j * g.ph;
+    for (int i = tid; i < g.kxr; i += NT) {
+      cx<T> A0, B0;
+      pair_split(s + pd * NX, i, NX, A0, B0);
+      if (pf >= 0) {
+        const T k = (T)kxt[i];
+        cx<T> A1, B1;
+        pair_split(s + (pf >= 0 ? pf : 0) * NX, i, NX, A1, B1);
+        A0 = cx<T>{k * A0.y, -(k * A0.x)} - A1;
+        B0 = cx<T>{k * B0.y, -(k * B0.x)} - B1;
+      }
+      H[(long long)z * g.kxp + i] = rnx * A0;
+      H[(long long)(z + 1) * g.kxp + i] = rnx * B0;
+    }
+  }
+}
+
+// The LES x pass: the closure, the products and their forward x transforms in one
+// kernel.  Block (z pair, plane j): every thread evaluates the model at its columns
+// of the two lines, one point after another, writes nu_t and kappa_t, and puts the
+// products with the SGS stresses added into the LDS lines (the pair's first line in
+// the real parts, the second in the imaginary ones).  The gradient fields are read
+// once; the 7 + 2 N_th SGS fields a separate model kernel wrote and the product
+// kernel read back never reach memory.  Planes follow one another on an XCD
+// (blocks b, b + 8, ...), so that the rows j - 1 .. j + 2 a block reads are in its L2.
+// Memory traffic bounds it in float; in FP64 the model's arithmetic and the
+// transforms cost as much, and the blocks of a CU overlap them.
+//
+// SPLIT: the lines of u1's and u3's equations are transformed first, those of u2's
+// and the scalars' held in registers meanwhile, so that the tile is half the size
+// and two or more blocks share a CU (where the whole tile leaves room for one, a
+// CU's loads, arithmetic and transforms run one after another).
+//
+// One launch, against the model and product kernels it replaces: 512x257x512 FP64
+// 6350 -> 4240 us (in one piece: 5505), float 2796 -> 2070; 128x129x128 FP64
+// (in one piece) 213 -> 115.
+template <typename T, int NX, int NT, int NTH, int MODEL, bool SPLIT>
+__global__ __launch_bounds__(NT) void k_les_products(XProdArgs x, AmdArgs a, int nj) {
+  constexpr int NP = 8 + 3 * NTH, NA = 5, NB = NP - NA;
+  constexpr int NL = SPLIT ? (NA > NB ? NA : NB) : NP;
+  constexpr int K = (2 * NX + NT - 1) / NT;  // points per thread
+  __shared__ cx<T> s[NL * NX];
+  __shared__ cx<T> stw[NX];  // twiddles
+  stage_twiddles<T, NX, NT>(stw, (const cx<T>*)x.tw, threadIdx.x);
+  const Geo& g = x.g;
+  const int tid = threadIdx.x, pairs = g.nz / 2;
+  int zp, jj;
+  xcd_rows(blockIdx.x, pairs, nj, zp, jj);
+  const int z = 2 * zp;
+  // one value to the compiler: the window's row differences fold to constants
+  const int j = __builtin_amdgcn_readfirstlane(x.jlo + jj);
+  T PB[SPLIT ? K : 1][NB];
+  // point c of the pair: line c / NX, column c mod NX
+  auto point = [&](int c, T* pb) __attribute__((always_inline)) {
+    const int xc = c & (NX - 1), line = c / NX;
+    const long long q = pcol(g, (long long)(z + line) * NX + xc), o = (long long)j * NX + q;
+    T win[3 * (3 + NTH)][4];
+    AmdIn<T> in;
+    in.w = win;
+    load_window<T, 3 * (3 + NTH)>(in, a, j, q);
+    AmdOut<T, NTH> r;
+    amd_point<T, NTH, MODEL>(in, a, j, q, r);
+    ((T*)a.nut)[o] = r.nut;
+#pragma unroll
+    for (int n = 0; n < NTH; ++n) ((T*)a.kap[n])[o] = r.kap[n];
+    T P[NP];
+    les_products<T, NTH>(x, in, j, r, P);
+    auto put = [&](int slot, T v) { ((T*)&s[slot * NX + swz<T>(xc)])[line] = v; };
+    if constexpr (SPLIT) {
+#pragma unroll
+      for (int p = 0; p < NA; ++p) put(p, P[les_line<NTH>(p)]);
+#pragma unroll
+      for (int p = 0; p < NB; ++p) pb[p] = P[les_line<NTH>(NA + p)];
+    } else {
+#pragma unroll
+      for (int p = 0; p < NP; ++p) put(p, P[p]);
+    }
+  };
+  if constexpr (SPLIT) {
+    static_assert(2 * NX == K * NT, "whole points");
+#pragma unroll
+    for (int k = 0; k < K; ++k) point(tid + k * NT, PB[k]);
+  } else {
+    for (int c = tid; c < 2 * NX; c += NT) point(c, PB[0]);
+  }
+  __syncthreads();
+  if constexpr (SPLIT) {
+    fft_lds_sync<T, NX, NA, NT, -1>(s, NX, stw, tid);
+    les_store<T, NX, NT, NTH, 0>(s, g, x.hout, x.kx, z, j, tid);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int c = tid + k * NT, xc = c & (NX - 1), line = c / NX;
+#pragma unroll
+      for (int p = 0; p < NB; ++p) ((T*)&s[p * NX + swz<T>(xc)])[line] = PB[k][p];
+    }
+    __syncthreads();
+    fft_lds_sync<T, NX, NB, NT, -1>(s, NX, stw, tid);
+    les_store<T, NX, NT, NTH, 1>(s, g, x.hout, x.kx, z, j, tid);
+  } else {
+    fft_lds_sync<T, NX, NP, NT, -1>(s, NX, stw, tid);
+    xprod_store<T, NX, NT, NTH>(s, g, x.hout, x.kx, z, j, tid);
   }
 }
 

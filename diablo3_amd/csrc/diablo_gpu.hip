@@ -115,7 +115,6 @@ struct dgpu_handle {
   void* Pg[3 * MAXF] = {};  // T
   void* NuT = nullptr;
   void* KapT[MAXTH] = {};
-  void* Aug[MAXA] = {};
   cd* CR[MAXF] = {};
   double* Rp[MAXF] = {};
   double* d_dlt = nullptr;  // [2][ny2]: delta_yf, delta_y of the AMD filter width
@@ -420,9 +419,9 @@ int ensure_fft_scratch(dgpu_handle* h) {
 // per-kernel timing
 // --------------------------------------------------------------------------------
 constexpr int NKERN = 13;
-const char* const kKernelNames[NKERN] = {"k_inv_z",   "k_xprod",  "k_fwdz_nl", "k_cn",      "k_project",
-                                         "k_bc_post", "les_grad", "k_amd",     "k_cn_phys", "les_cn_fft",
-                                         "k_closure", "k_xmarch", "k_column"};
+const char* const kKernelNames[NKERN] = {"k_inv_z",   "k_les_products", "k_fwdz_nl", "k_cn",      "k_project",
+                                         "k_bc_post", "les_grad",       "",          "k_cn_phys", "les_cn_fft",
+                                         "k_closure", "k_xmarch",       "k_column"};
 
 hipEvent_t pool_event(dgpu_handle* h) {
   if (!h->ev_pool.empty()) {
@@ -486,8 +485,8 @@ int launch_inv_z(dgpu_handle* h, int nf, const cd* const* src, void* const* dst,
   const cx<T>* tw = (const cx<T>*)(sizeof(T) == 8 ? h->twz64 : h->twz32);
   DG_SWITCH_N(h->g.nz, {
     constexpr int TI = ti_for(N_, sizeof(cx<T>));
-    dim3 grid((h->g.kxr + TI - 1) / TI, nj, nf);
-    k_inv_z<T, N_, TI, 256><<<grid, 256, 0, h->st>>>(s, d, h->g, j0, tw, h->d_kz, dzmask);
+    const int grid = batch_grid((h->g.kxr + TI - 1) / TI * nj, nf, ZK<T, TI>);
+    k_inv_z<T, N_, TI, 256><<<grid, 256, 0, h->st>>>(s, d, h->g, j0, nj, nf, tw, h->d_kz, dzmask);
   });
   HIPCHK(hipGetLastError());
   return 0;
@@ -562,25 +561,24 @@ int launch_fwd_x(dgpu_handle* h, int nf, const T* const* src, void* const* dst, 
   return 0;
 }
 
-// threads per k_xprod block: 256 for the larger lines; where the LDS tile
-// (> 80 KiB) leaves room for one block per CU only, one thread per column of
-// the line (up to 1024), so that a CU still holds 8 or 16 waves
-constexpr int xprod_nt(int nx, size_t lds) {
-  return nx <= 32 ? 64 : (nx == 64 ? 128 : (lds > 81920 ? (nx >= 1024 ? 1024 : 512) : 256));
-}
+// threads per k_les_products block
+constexpr int les_nt(int nx) { return nx <= 32 ? 64 : (nx == 64 ? 128 : 256); }
 
-template <typename T, int NTH, bool LES = false>
-int launch_xprod(dgpu_handle* h, XProdArgs& a, int nj) {
-  a.tw = sizeof(T) == 8 ? h->twx64 : h->twx32;
+template <typename T, int NTH, int MODEL>
+int launch_les_products(dgpu_handle* h, XProdArgs& x, const AmdArgs& a, int nj) {
+  x.tw = sizeof(T) == 8 ? h->twx64 : h->twx32;
   DG_SWITCH_N(h->g.nx, {
     // product lines + twiddle table
     constexpr size_t lds = sizeof(cx<T>) * ((8 + 3 * NTH) + 1) * N_;
     if constexpr (lds > 163840) {
       return fail(2, "this nx needs the mixed-precision mode (x pass exceeds LDS in FP64)");
     } else {
-      constexpr int NT = xprod_nt(N_, lds);
-      dim3 grid(h->g.nz / 2, nj, 1);
-      k_xprod<T, N_, NT, NTH, LES><<<grid, NT, 0, h->st>>>(a);
+      // the tile in two halves where the whole one (> 80 KiB) leaves room for one
+      // block per CU only (512 lines FP64: 5505 us in one piece, 4240 in two); below,
+      // two or more blocks fit as it is and the halves only add barriers
+      constexpr int NT = les_nt(N_);
+      k_les_products<T, N_, NT, NTH, MODEL, (lds > 81920)>
+          <<<(unsigned)(h->g.nz / 2 * nj), NT, 0, h->st>>>(x, a, nj);
     }
   });
   HIPCHK(hipGetLastError());
@@ -817,12 +815,15 @@ int physical_gradients(dgpu_handle* h, void* const* H, void* const* HZ, void* co
   const int nf = 3 + h->nth;
   const cd* zs[2 * MAXF];
   void* zd[2 * MAXF];
+  unsigned dzmask = 0;
+  // v beside dv/dz: k_inv_z reads their common source once
   for (int f = 0; f < nf; ++f) {
-    zs[f] = h->U[f]; zd[f] = H[f];
-    zs[nf + f] = h->U[f]; zd[nf + f] = HZ[f];
+    zs[2 * f] = h->U[f]; zd[2 * f] = H[f];
+    zs[2 * f + 1] = h->U[f]; zd[2 * f + 1] = HZ[f];
+    dzmask |= 2u << (2 * f);
   }
   int rc;
-  if ((rc = launch_inv_z<T>(h, 2 * nf, zs, zd, 0, g.ny2, ((1u << nf) - 1u) << nf))) return rc;
+  if ((rc = launch_inv_z<T>(h, 2 * nf, zs, zd, 0, g.ny2, dzmask))) return rc;
   void* xs[3 * MAXF];
   T* xd[3 * MAXF];
   unsigned dxmask = 0;
@@ -974,7 +975,7 @@ int substep_les(dgpu_handle* h, int rk, double delta_t, double time, int time_st
   if ((rc = physical_gradients<T>(h, h->Hin, h->HinZ, h->Pg))) return rc;
   if ((rc = tend(h))) return rc;
 
-  // 2. AMD: nu_t, kappa_t and the SGS additions to the products
+  // 2. the model's arguments
   AmdArgs aa{};
   aa.g = g; aa.nth = NTH; aa.jstart = c.jstart; aa.jend = c.jend;
   for (int n = 0; n < MAXTH; ++n) { aa.jstart_th[n] = c.jstart_th[n]; aa.jend_th[n] = c.jend_th[n]; }
@@ -984,7 +985,6 @@ int substep_les(dgpu_handle* h, int rk, double delta_t, double time, int time_st
   for (int s = 0; s < 3 * nf; ++s) aa.f[s] = h->Pg[s];
   aa.nut = h->NuT;
   for (int n = 0; n < NTH; ++n) aa.kap[n] = h->KapT[n];
-  for (int m = 0; m < 7 + 2 * NTH; ++m) aa.aug[m] = h->Aug[m];
   // one block per (256 points, row): xcd_rows maps the 1D index
   const dim3 agrid((unsigned)(((g.pp + 255) / 256) * g.ny2));
   if constexpr (NTH == 1) {
@@ -998,29 +998,22 @@ int substep_les(dgpu_handle* h, int rk, double delta_t, double time, int time_st
       aa.cgy = h->Cgy; aa.kgy = h->Kgy;
     }
   }
-  if ((rc = tbeg(h, 7))) return rc;
-  if (c.les_model_type == 1) k_amd<T, NTH, 1><<<agrid, 256, 0, h->st>>>(aa);
-  else if (c.les_model_type == 4) k_amd<T, NTH, 4><<<agrid, 256, 0, h->st>>>(aa);
-  else if (c.les_model_type == 6 && NTH == 1) k_amd<T, NTH, 6><<<agrid, 256, 0, h->st>>>(aa);
-  else k_amd<T, NTH, 5><<<agrid, 256, 0, h->st>>>(aa);
-  HIPCHK(hipGetLastError());
-  if ((rc = tend(h))) return rc;
 
-  // 3. fused x pass: products + SGS stresses; 4. z forward -> nonlinear tendencies
+  // 3. fused x pass: the model, products + SGS stresses; 4. z forward -> nonlinear
+  //    tendencies
   XProdArgs xa{};
   xa.g = g; xa.jlo = jlo; xa.jstart = c.jstart; xa.jend = c.jend;
   for (int n = 0; n < MAXTH; ++n) { xa.jstart_th[n] = c.jstart_th[n]; xa.jend_th[n] = c.jend_th[n]; }
   xa.dy = h->d_dy; xa.dyf = h->d_dyf; xa.kx = h->d_kx; xa.rowc = h->d_rowc;
   for (int f = 0; f < nf; ++f) xa.hin[f] = h->Hin[f];
   for (int o = 0; o < 6 + 2 * NTH; ++o) xa.hout[o] = h->Hout[o];
-  for (int m = 0; m < 7 + 2 * NTH; ++m) xa.aug[m] = h->Aug[m];
-  for (int f = 0; f < nf; ++f) {
-    xa.phys[f] = h->Pg[3 * f];  // the gradient stage's physical fields
-    if (!xa.phys[f]) return fail(12, "x pass: physical field buffer missing");
-  }
   if ((rc = tbeg(h, 1))) return rc;
-  if ((rc = launch_xprod<T, NTH, true>(h, xa, nj))) return rc;
-  if ((rc = tend(h))) return rc;
+  if (c.les_model_type == 1) rc = launch_les_products<T, NTH, 1>(h, xa, aa, nj);
+  else if (c.les_model_type == 4) rc = launch_les_products<T, NTH, 4>(h, xa, aa, nj);
+  else if constexpr (NTH == 1) rc = c.les_model_type == 6 ? launch_les_products<T, NTH, 6>(h, xa, aa, nj)
+                                                          : launch_les_products<T, NTH, 5>(h, xa, aa, nj);
+  else rc = launch_les_products<T, NTH, 5>(h, xa, aa, nj);
+  if (rc || (rc = tend(h))) return rc;
   NlArgs na{};
   na.g = g; na.jlo = jlo; na.jstart = c.jstart; na.jend = c.jend;
   for (int n = 0; n < MAXTH; ++n) { na.jstart_th[n] = c.jstart_th[n]; na.jend_th[n] = c.jend_th[n]; }
@@ -1300,7 +1293,6 @@ int dgpu_create(const dgpu_config* cfg, dgpu_handle** out) {
     }
     ALLOC(h->NuT, tbytes);
     for (int n = 0; n < h->nth; ++n) ALLOC(h->KapT[n], tbytes);
-    for (int m = 0; m < 7 + 2 * h->nth; ++m) ALLOC(h->Aug[m], tbytes);
     ALLOC(h->d_dlt, sizeof(double) * 2 * n2);
     if (cfg->les_model_type == 6) {
       ALLOC(h->Cgy, tbytes);

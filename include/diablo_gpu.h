@@ -181,10 +181,10 @@ int dgpu_last_step_ms(dgpu_handle *h, double *ms);
 /* Per-kernel device timing, for measurement only (no counterpart in the
  * reference).  While enabled, every launch of the step's kernels is bracketed by
  * HIP events on the handle's stream.  Kernel ids: 0 = z inverse transform of the
- * state, 1 = the LES x pass (products), 2 = z forward transform of the products,
- * 3 = Fourier assembly (LES; with the Crank-Nicolson solves where courant follows
+ * state, 1 = the LES x pass (model, products and their forward x
+ * transforms), 2 = z forward transform of the products, 3 = Fourier assembly (LES; with the Crank-Nicolson solves where courant follows
  * them in a DNS substep), 4 = projection + pressure update (LES, and after courant);
- * LES substeps add 5 = BC posts, 6 = gradient fields, 7 = AMD model,
+ * LES substeps add 5 = BC posts, 6 = gradient fields, 7 = not used,
  * 8 = physical-column CN solves, 9 = right-hand-side and solution transforms,
  * 10 = the learned closure's coefficients (les_model_type 6, dgpu_closure.h),
  * 11 = the DNS x pass (x inverse transforms, products and x forward transforms
