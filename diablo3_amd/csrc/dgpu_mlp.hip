@@ -18,15 +18,28 @@ static_assert(DGPU_MLP_NNORM == MLP_NNORM, "normaliser size");
 
 namespace dgpu {
 
+// offsets of the BF16 weight copies (in elements; each a multiple of 4, so
+// every 4-element operand load is 8-byte aligned)
+constexpr int WB_W1T = 0, WB_W2T = WB_W1T + 64 * 16, WB_W3T = WB_W2T + 64 * 64, WB_W2 = WB_W3T + 16 * 64,
+              WB_W3 = WB_W2 + 64 * 64, WB_N = WB_W3 + 64 * 16;
+
 // ---------------------------------------------------------------------------
 // Training: the gradient of the minibatch loss
 //   L = (1/n) sum_s sum_o wo_o (y_so - t_so)^2
 // One block (4 waves) accumulates its tiles in registers; the waves' sums are
 // added in a fixed order in LDS and written as the block's partial gradient,
 // so the result does not depend on scheduling (no atomics).
+//
+// A minibatch gives a wave a tile or two, so latency bounds it: the weights come to
+// LDS in one round of loads at the start (as operands read from memory where they
+// were used, each waited for the last), a tile's samples are read one tile ahead,
+// and the four waves' turns at the sum overlap.  Per minibatch of 16384 (256
+// blocks): 24 -> 15 us; of 1024: 22 -> 12.5.
 // ---------------------------------------------------------------------------
 struct MlpGradArgs {
-  MlpW w;
+  const unsigned short* wb;  // the BF16 weight copies
+  const float* p;            // FP32 master parameters (the biases)
+  const float* norm;
   const float* X;    // [N][16] raw features
   const float* T;    // [N][2] targets
   const int* idx;    // minibatch sample indices (null: samples 0..n-1)
@@ -38,11 +51,47 @@ struct MlpGradArgs {
 
 __device__ __forceinline__ long long mlp_row(const int* idx, long long s) { return idx ? (long long)idx[s] : s; }
 
+// The block's sums in LDS: the parameter block with its rows padded by four, so that
+// the 16 rows a wave's tile touches start in different banks.
+constexpr int RED_LD = MLP_H + 4, RED_LD3 = MLP_OUTP + 4;
+constexpr int RED_W1 = 0, RED_B1 = RED_W1 + MLP_INP * RED_LD, RED_W2 = RED_B1 + MLP_H, RED_B2 = RED_W2 + MLP_H * RED_LD,
+              RED_W3 = RED_B2 + MLP_H, RED_B3 = RED_W3 + MLP_H * RED_LD3, RED_N = RED_B3 + MLP_OUTP;
+// where parameter i is (four consecutive ones from a multiple of 4 stay together)
+__device__ __forceinline__ int red_slot(int i) {
+  if (i < MLP_OB1) return RED_W1 + i + 4 * (i / MLP_H);
+  if (i < MLP_OW2) return RED_B1 + i - MLP_OB1;
+  if (i < MLP_OB2) return RED_W2 + (i - MLP_OW2) + 4 * ((i - MLP_OW2) / MLP_H);
+  if (i < MLP_OW3) return RED_B2 + i - MLP_OB2;
+  if (i < MLP_OB3) return RED_W3 + (i - MLP_OW3) + 4 * ((i - MLP_OW3) / MLP_OUTP);
+  return RED_B3 + i - MLP_OB3;
+}
+// sum over the 16 lanes of a row: pairs 8, 4, 2 and 1 apart (a rotation by 8, 4, 2, 1
+// reaches the same partner, the values having that period by then)
+__device__ __forceinline__ float row16_sum(float x) {
+#define DG_ROR(n) x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x120 + n, 0xf, 0xf, true))
+  DG_ROR(8); DG_ROR(4); DG_ROR(2); DG_ROR(1);
+#undef DG_ROR
+  return x;
+}
+
+// The BF16 weights in LDS: rows of 64 padded by four (16 rows of a wave's operand
+// load start in different banks); rows of 16 as they are.
+constexpr int SW_LD = MLP_H + 4;
+constexpr int SW_W1T = 0, SW_W2T = SW_W1T + 64 * 16, SW_W3T = SW_W2T + 64 * SW_LD, SW_W2 = SW_W3T + 16 * SW_LD,
+              SW_W3 = SW_W2 + 64 * SW_LD, SW_N = SW_W3 + 64 * 16;
+// where element i (a multiple of 8) of the weight copies goes
+__device__ __forceinline__ int sw_slot(int i) {
+  if (i < WB_W2T || i >= WB_W3) return i < WB_W2T ? SW_W1T + i : SW_W3 + i - WB_W3;
+  return SW_W2T + (i - WB_W2T) + 4 * ((i - WB_W2T) / MLP_H);  // w2t, w3t, w2: 144 rows of 64
+}
+
 __global__ __launch_bounds__(256) void k_mlp_grad(MlpGradArgs a) {
   __shared__ unsigned short sA[4][64 * 16];  // per wave: [neuron][sample] transposes
   __shared__ unsigned short sB[4][64 * 16];
-  __shared__ float red[MLP_NP];
+  __shared__ __attribute__((aligned(16))) float red[RED_N];
   __shared__ float sred[256];
+  __shared__ __attribute__((aligned(16))) unsigned short sw[SW_N];
+  __shared__ float sb[2 * MLP_H + MLP_OUTP], sn[2 * MLP_INP];
   const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, r = l & 15, g = l >> 4;
   unsigned short* TA = sA[wave];
   unsigned short* TB = sB[wave];
@@ -58,20 +107,55 @@ __global__ __launch_bounds__(256) void k_mlp_grad(MlpGradArgs a) {
   }
   gb3 = zero4;
   float lsum = 0.f;
-  const long long ntile = (a.n + 15) / 16;
+  const long long ntile = (a.n + 15) / 16, stride = (long long)gridDim.x * 4;
+  long long t = (long long)blockIdx.x * 4 + wave;
+  // a tile's sample of this lane (0 past the last), and its features 4g..4g+3 and
+  // targets: read one tile ahead, the index two
+  auto row_of = [&](long long tt) { return tt * 16 + r < a.n ? mlp_row(a.idx, tt * 16 + r) : 0; };
+  const long long row0 = row_of(t);
+  float4 x = *(const float4*)(a.X + row0 * MLP_INP + 4 * g);
+  float2 tg = *(const float2*)(a.T + row0 * 2);
+  long long row = row_of(t + stride);
+  // the weights, biases and normaliser in LDS, every load in flight at once
+  {
+    constexpr int PER = (WB_N / 8 + 255) / 256;
+    uint4 t[PER];
+    float b = 0.f, nr = 0.f;
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) t[k] = ((const uint4*)a.wb)[min(tid + 256 * k, WB_N / 8 - 1)];
+    if (tid < 2 * MLP_H + MLP_OUTP)
+      b = a.p[tid < MLP_H ? MLP_OB1 + tid : (tid < 2 * MLP_H ? MLP_OB2 + tid - MLP_H : MLP_OB3 + tid - 2 * MLP_H)];
+    if (tid < 2 * MLP_INP) nr = a.norm[tid];
+#pragma unroll
+    for (int k = 0; k < PER; ++k)
+      if (tid + 256 * k < WB_N / 8) {
+        uint2* q = (uint2*)&sw[sw_slot(8 * (tid + 256 * k))];
+        q[0] = uint2{t[k].x, t[k].y};
+        q[1] = uint2{t[k].z, t[k].w};
+      }
+    if (tid < 2 * MLP_H + MLP_OUTP) sb[tid] = b;
+    if (tid < 2 * MLP_INP) sn[tid] = nr;
+  }
+  __syncthreads();
+  MlpW w;
+  w.w1t = sw + SW_W1T; w.w2t = sw + SW_W2T; w.w3t = sw + SW_W3T; w.w2 = sw + SW_W2; w.w3 = sw + SW_W3;
+  w.b1 = sb; w.b2 = sb + MLP_H; w.b3 = sb + 2 * MLP_H; w.norm = sn;
   const float inv_n = 1.0f / (float)a.n;
-  for (long long t = (long long)blockIdx.x * 4 + wave; t < ntile; t += (long long)gridDim.x * 4) {
-    const long long s = t * 16 + r;
-    const bool live = s < a.n;
-    const long long row = live ? mlp_row(a.idx, s) : 0;
-    bf16x4 xb = norm_x(a.w.norm, a.X + row * MLP_INP + 4 * g, g);
+  for (; t < ntile; t += stride) {
+    const bool live = t * 16 + r < a.n;
+    const float t0 = tg.x, t1 = tg.y;
+    bf16x4 xb = norm_x(w.norm, &x.x, g);
+    x = *(const float4*)(a.X + row * MLP_INP + 4 * g);
+    tg = *(const float2*)(a.T + row * 2);
+    row = row_of(t + 2 * stride);
     if (!live) xb = bf16x4{0, 0, 0, 0};
     MlpAct act;
-    mlp_forward(a.w, xb, act);
+    mlp_forward<SW_LD>(w, xb, act);
     // dL/dy in the accumulator layout (rows = outputs 4g+v, column = sample r)
     f32x4 dy = zero4;
     if (g == 0 && live) {
-      const float e0 = act.y[0] - a.T[row * 2], e1 = act.y[1] - a.T[row * 2 + 1];
+      const float e0 = act.y[0] - t0, e1 = act.y[1] - t1;
       lsum += a.wo0 * e0 * e0 + a.wo1 * e1 * e1;
       dy[0] = 2.f * a.wo0 * e0 * inv_n;
       dy[1] = 2.f * a.wo1 * e1 * inv_n;
@@ -97,7 +181,7 @@ __global__ __launch_bounds__(256) void k_mlp_grad(MlpGradArgs a) {
     bf16x4 dz2b[4];
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) {
-      f32x4 c = mfma16(ld4(a.w.w3 + (kb * 16 + r) * MLP_OUTP + 4 * g), dyb, zero4);
+      f32x4 c = mfma16(ld4(w.w3 + (kb * 16 + r) * MLP_OUTP + 4 * g), dyb, zero4);
 #pragma unroll
       for (int v = 0; v < 4; ++v) c[v] *= dgelu(act.z2[kb][v]);
       dz2[kb] = c;
@@ -126,7 +210,7 @@ __global__ __launch_bounds__(256) void k_mlp_grad(MlpGradArgs a) {
     for (int kb = 0; kb < 4; ++kb) {
       f32x4 c = zero4;
 #pragma unroll
-      for (int ob = 0; ob < 4; ++ob) c = mfma16(ld4(a.w.w2 + (kb * 16 + r) * MLP_H + ob * 16 + 4 * g), dz2b[ob], c);
+      for (int ob = 0; ob < 4; ++ob) c = mfma16(ld4(w.w2 + (kb * 16 + r) * SW_LD + ob * 16 + 4 * g), dz2b[ob], c);
 #pragma unroll
       for (int v = 0; v < 4; ++v) c[v] *= dgelu(act.z1[kb][v]);
       dz1[kb] = c;
@@ -153,59 +237,50 @@ __global__ __launch_bounds__(256) void k_mlp_grad(MlpGradArgs a) {
 #pragma unroll
   for (int ob = 0; ob < 4; ++ob)
 #pragma unroll
-    for (int v = 0; v < 4; ++v)
-#pragma unroll
-      for (int m = 8; m >= 1; m >>= 1) {
-        gb1[ob][v] += __shfl_xor(gb1[ob][v], m, 16);
-        gb2[ob][v] += __shfl_xor(gb2[ob][v], m, 16);
-      }
-#pragma unroll
-  for (int v = 0; v < 4; ++v)
-#pragma unroll
-    for (int m = 8; m >= 1; m >>= 1) gb3[v] += __shfl_xor(gb3[v], m, 16);
-  // the waves add their sums into red[] one after another (W^T tiles hold
-  // [out][in]; the parameter block stores W as [in][out])
-  for (int i = threadIdx.x; i < MLP_NP; i += 256) red[i] = 0.f;
-  __syncthreads();
-  for (int wv = 0; wv < 4; ++wv) {
-    if (wave == wv) {
-#pragma unroll
-      for (int ob = 0; ob < 4; ++ob)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) red[MLP_OW1 + r * MLP_H + ob * 16 + 4 * g + v] += gw1[ob][v];
-#pragma unroll
-      for (int ob = 0; ob < 4; ++ob)
-#pragma unroll
-        for (int ib = 0; ib < 4; ++ib)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) red[MLP_OW2 + (ib * 16 + r) * MLP_H + ob * 16 + 4 * g + v] += gw2[ob][ib][v];
-#pragma unroll
-      for (int ib = 0; ib < 4; ++ib)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) red[MLP_OW3 + (ib * 16 + r) * MLP_OUTP + 4 * g + v] += gw3[ib][v];
-      if (r == 0) {
-#pragma unroll
-        for (int ob = 0; ob < 4; ++ob)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            red[MLP_OB1 + ob * 16 + 4 * g + v] += gb1[ob][v];
-            red[MLP_OB2 + ob * 16 + 4 * g + v] += gb2[ob][v];
-          }
-#pragma unroll
-        for (int v = 0; v < 4; ++v) red[MLP_OB3 + 4 * g + v] += gb3[v];
-      }
+    for (int v = 0; v < 4; ++v) {
+      gb1[ob][v] = row16_sum(gb1[ob][v]);
+      gb2[ob][v] = row16_sum(gb2[ob][v]);
     }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) gb3[v] = row16_sum(gb3[v]);
+  // The waves add their sums into red[] one after another (W^T tiles hold
+  // [out][in]; the parameter block stores W as [in][out]), a quarter of the
+  // parameters behind one another: wave w adds quarter ob in step w + ob.
+#pragma unroll
+  for (int step = 0; step < 7; ++step) {
+#pragma unroll
+    for (int ob = 0; ob < 4; ++ob)
+      if (wave == step - ob) {
+        const f32x4 x[9] = {gw1[ob], gw2[ob][0], gw2[ob][1], gw2[ob][2], gw2[ob][3], gw3[ob], gb1[ob], gb2[ob], gb3};
+        f32x4* q[9];
+        q[0] = (f32x4*)&red[RED_W1 + r * RED_LD + ob * 16 + 4 * g];
+#pragma unroll
+        for (int ib = 0; ib < 4; ++ib) q[1 + ib] = (f32x4*)&red[RED_W2 + (ib * 16 + r) * RED_LD + ob * 16 + 4 * g];
+        q[5] = (f32x4*)&red[RED_W3 + (ob * 16 + r) * RED_LD3 + 4 * g];
+        // (the 16 lanes of a row hold the same bias sums)
+        q[6] = (f32x4*)&red[RED_B1 + ob * 16 + 4 * g];
+        q[7] = (f32x4*)&red[RED_B2 + ob * 16 + 4 * g];
+        q[8] = (f32x4*)&red[RED_B3 + 4 * g];
+        f32x4 o[9];
+#pragma unroll
+        for (int k = 0; k < (ob == 0 ? 9 : 8); ++k) o[k] = wave == 0 ? zero4 : *q[k];
+#pragma unroll
+        for (int k = 0; k < (ob == 0 ? 9 : 8); ++k) o[k] += x[k];
+#pragma unroll
+        for (int k = 0; k < (ob == 0 ? 9 : 8); ++k) *q[k] = o[k];
+      }
+    if (step == 0) sred[threadIdx.x] = lsum;
     __syncthreads();
   }
   float* P = a.part + (long long)blockIdx.x * MLP_NP;
-  for (int i = threadIdx.x; i < MLP_NP; i += 256) P[i] = red[i];
-  sred[threadIdx.x] = lsum;
-  __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if ((int)threadIdx.x < st) sred[threadIdx.x] += sred[threadIdx.x + st];
-    __syncthreads();
+  for (int i = 4 * threadIdx.x; i < MLP_NP; i += 1024) *(f32x4*)(P + i) = *(const f32x4*)&red[red_slot(i)];
+  // the block's loss: halves of the 256 threads' sums added to each other
+  if (wave == 0) {
+    float x = (sred[l] + sred[l + 128]) + (sred[l + 64] + sred[l + 192]);
+#pragma unroll
+    for (int st = 32; st > 0; st >>= 1) x += __shfl_down(x, st);
+    if (l == 0) a.lpart[blockIdx.x] = x;
   }
-  if (threadIdx.x == 0) a.lpart[blockIdx.x] = sred[0];
 }
 
 // Sum of the partial gradients (fixed order), then either the gradient out
@@ -251,27 +326,61 @@ __device__ __forceinline__ void mlp_store_bf16(const MlpAdamArgs& a, int i, floa
   }
 }
 
+// Latency bounds it: one thread per parameter reading its partials one after another
+// took 66 us for 256 of them.  Here a block takes ADAM_P parameters (a 128-byte line
+// of each partial), 256 threads bring ADAM_ROWS partials at a time to LDS in one
+// round of loads, and one thread per parameter adds them in the same order: 5.4 us.
+constexpr int ADAM_P = 32, ADAM_ROWS = 128;
 __global__ __launch_bounds__(256) void k_mlp_adam(MlpAdamArgs a) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i == 0 && a.loss) {
-    float s = 0.f;
-    for (int b = 0; b < a.nblk; ++b) s += a.lpart[b];
-    *a.loss += s * a.lscale;
+  __shared__ float s[2][ADAM_ROWS * ADAM_P];
+  __shared__ float sl[256];
+  const int tid = threadIdx.x, c = tid % ADAM_P, rg = tid / ADAM_P, i0 = blockIdx.x * ADAM_P, i = i0 + c;
+  const bool in = i < MLP_NP, sum = tid < ADAM_P && in;
+  // the master values of the parameters, on their way while the partials are read
+  float pm = 0.f, pv = 0.f, pp = 0.f;
+  if (sum && a.mode) { pm = a.m[i]; pv = a.v[i]; pp = a.p[i]; }
+  const bool loss = blockIdx.x == 0 && a.loss;
+  constexpr int PER = ADAM_ROWS * ADAM_P / 256;
+  // rows b0.. of the partials into registers (zero past the last: adding one changes
+  // no sum that began at zero)
+  float x[PER];
+  auto load = [&](int b0) {
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int b = b0 + rg + k * (256 / ADAM_P);
+      x[k] = in && b < a.nblk ? a.part[(long long)b * MLP_NP + i] : 0.f;
+    }
+  };
+  float gr = 0.f, ls = 0.f;
+  load(0);
+  for (int b0 = 0, buf = 0; b0 < a.nblk; b0 += ADAM_ROWS, buf ^= 1) {
+#pragma unroll
+    for (int k = 0; k < PER; ++k) s[buf][(rg + k * (256 / ADAM_P)) * ADAM_P + c] = x[k];
+    if (loss && tid < ADAM_ROWS) sl[buf * ADAM_ROWS + tid] = b0 + tid < a.nblk ? a.lpart[b0 + tid] : 0.f;
+    __syncthreads();
+    if (b0 + ADAM_ROWS < a.nblk) load(b0 + ADAM_ROWS);
+    const int rows = (min(ADAM_ROWS, a.nblk - b0) + 15) / 16 * 16;
+    if (tid < ADAM_P) {
+      for (int r = 0; r < rows; r += 16)
+#pragma unroll
+        for (int k = 0; k < 16; ++k) gr += s[buf][(r + k) * ADAM_P + c];
+    } else if (loss && tid == 64) {
+      for (int r = 0; r < rows; ++r) ls += sl[buf * ADAM_ROWS + r];
+    }
   }
-  if (i >= MLP_NP) return;
-  float gr = 0.f;
-  for (int b = 0; b < a.nblk; ++b) gr += a.part[(long long)b * MLP_NP + i];
+  if (loss && tid == 64) *a.loss += ls * a.lscale;
+  if (!sum) return;
   if (a.mode == 0) {
     a.grad[i] = gr;
     return;
   }
   float w = 0.f;
   if (mlp_param_live(i)) {
-    const float m = a.b1 * a.m[i] + (1.f - a.b1) * gr;
-    const float v = a.b2 * a.v[i] + (1.f - a.b2) * gr * gr;
+    const float m = fmaf(1.f - a.b1, gr, a.b1 * pm);
+    const float v = fmaf(gr, (1.f - a.b2) * gr, a.b2 * pv);
     a.m[i] = m;
     a.v[i] = v;
-    w = a.p[i] - a.lr * (m * a.c1) / (sqrtf(v * a.c2) + a.eps);
+    w = pp - a.lr * (m * a.c1) / (sqrtf(v * a.c2) + a.eps);
   }
   a.p[i] = w;
   mlp_store_bf16(a, i, w);
@@ -317,10 +426,6 @@ namespace {
     if (e_ != hipSuccess) return set_error(10, std::string(#x) + ": " + hipGetErrorString(e_)); \
   } while (0)
 
-// offsets of the BF16 weight copies (in elements; each a multiple of 4, so
-// every 4-element operand load is 8-byte aligned)
-constexpr int WB_W1T = 0, WB_W2T = WB_W1T + 64 * 16, WB_W3T = WB_W2T + 64 * 64, WB_W2 = WB_W3T + 16 * 64,
-              WB_W3 = WB_W2 + 64 * 64, WB_N = WB_W3 + 64 * 16;
 constexpr int MAX_BLK = 512;
 
 uint64_t splitmix(uint64_t& s) {
@@ -402,7 +507,7 @@ int grad_blocks(long long n) {
 
 int launch_grad(dgpu_mlp* m, const int* idx, long long n, const float loss_w[2], int& nblk) {
   MlpGradArgs a{};
-  a.w = m->weights();
+  a.wb = m->wb; a.p = m->p; a.norm = m->norm;
   a.X = m->X; a.T = m->T; a.idx = idx; a.n = n;
   a.wo0 = loss_w ? loss_w[0] : 1.f;
   a.wo1 = loss_w ? loss_w[1] : 1.f;
@@ -423,7 +528,7 @@ int launch_adam(dgpu_mlp* m, int nblk, float lr, float* loss, float lscale) {
   a.lr = lr;
   a.c1 = (float)(1.0 / (1.0 - std::pow((double)m->b1, (double)m->t)));
   a.c2 = (float)(1.0 / (1.0 - std::pow((double)m->b2, (double)m->t)));
-  k_mlp_adam<<<(MLP_NP + 255) / 256, 256, 0, m->st>>>(a);
+  k_mlp_adam<<<(MLP_NP + ADAM_P - 1) / ADAM_P, 256, 0, m->st>>>(a);
   MCHK(hipGetLastError());
   return 0;
 }
@@ -528,7 +633,7 @@ int dgpu_mlp_grad(dgpu_mlp* m, int64_t n, const float loss_w[2], float* grad, fl
   MlpAdamArgs a = m->adam_args();
   a.nblk = nblk;
   a.mode = 0;
-  k_mlp_adam<<<(MLP_NP + 255) / 256, 256, 0, m->st>>>(a);
+  k_mlp_adam<<<(MLP_NP + ADAM_P - 1) / ADAM_P, 256, 0, m->st>>>(a);
   MCHK(hipGetLastError());
   MCHK(hipMemcpyAsync(grad, m->grad, sizeof(float) * MLP_NP, hipMemcpyDeviceToHost, m->st));
   std::vector<float> lp(nblk);

@@ -101,7 +101,8 @@ struct MlpAct {
 };
 
 // xb: the normalised input tile in B layout (lane l holds features 4*(l/16)+v
-// of sample l%16)
+// of sample l%16); LD: distance of the rows of 64 weights
+template <int LD>
 __device__ __forceinline__ void mlp_forward(const MlpW& w, bf16x4 xb, MlpAct& a) {
   const int l = threadIdx.x & 63, r = l & 15, g = l >> 4;
 #pragma unroll
@@ -122,7 +123,7 @@ __device__ __forceinline__ void mlp_forward(const MlpW& w, bf16x4 xb, MlpAct& a)
 #pragma unroll
     for (int v = 0; v < 4; ++v) c[v] = w.b2[ob * 16 + 4 * g + v];
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) c = mfma16(ld4(w.w2t + (ob * 16 + r) * MLP_H + kb * 16 + 4 * g), a.h1[kb], c);
+    for (int kb = 0; kb < 4; ++kb) c = mfma16(ld4(w.w2t + (ob * 16 + r) * LD + kb * 16 + 4 * g), a.h1[kb], c);
     a.z2[ob] = c;
     f32x4 h;
 #pragma unroll
@@ -133,7 +134,7 @@ __device__ __forceinline__ void mlp_forward(const MlpW& w, bf16x4 xb, MlpAct& a)
 #pragma unroll
   for (int v = 0; v < 4; ++v) c[v] = w.b3[4 * g + v];
 #pragma unroll
-  for (int kb = 0; kb < 4; ++kb) c = mfma16(ld4(w.w3t + r * MLP_H + kb * 16 + 4 * g), a.h2[kb], c);
+  for (int kb = 0; kb < 4; ++kb) c = mfma16(ld4(w.w3t + r * LD + kb * 16 + 4 * g), a.h2[kb], c);
   a.y = c;
 }
 
