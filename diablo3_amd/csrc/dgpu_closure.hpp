@@ -118,7 +118,7 @@ __device__ __forceinline__ GyEntries<T> gy_entries(const AmdIn<T>& in, const Amd
   using R = T;
   const Gyf<T> f = gyf_plane(in, a, j, q), fm = gyf_plane(in, a, j - 1, q);
   const Gy<T> p = gy_plane(in, a, j, q);
-  auto w = [&](R x, R y) { return gy_interp(a, j, x, y); };
+  auto w = [&](R x, R y) { return gy_interp(in, j, x, y); };
   return {w(f.a1, fm.a1), w(f.a2, fm.a2), w(f.a3, fm.a3), p.a4, w(f.a5, fm.a5), p.a6, p.o4, w(f.o5, fm.o5), p.o6};
 }
 
@@ -134,9 +134,13 @@ __global__ __launch_bounds__(256) void k_closure(ClosureArgs c) {
   const bool live = q0 < g.pp;
   const long long qf = live ? q0 : g.pp - 1, q = pcol(g, qf);  // every lane takes part in the MFMA tiles
   const int ny = g.ny;
-  T win[3 * (3 + NTH)][4];
+  T win[3 * (3 + NTH)][4], rows[3][K_N];
+  load_rows<T>(rows, a, j);
   AmdIn<T> in;
   in.w = win;
+  in.k = rows;
+  in.j0 = j - 1;
+  in.nx = g.nx;
   load_window<T, 3 * (3 + NTH)>(in, a, j, q);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   // step mode: GY rows 2..Nyp; feature mode: GYF rows jf0..Nyp-1

@@ -23,6 +23,8 @@
 #pragma once
 #include "dgpu_kernels.hpp"
 
+#include <type_traits>
+
 namespace dgpu {
 
 constexpr double C_AMD = 0.2887;     // for/les.f90:25
@@ -159,43 +161,58 @@ struct Gy {
   R a4, o4, a6, o6;
 };
 
+// What the model takes from the grid at one row: the quotients of the row table
+// (RowCoef), the filter widths and the spacings.  The reference divides by dy(j),
+// dyf(j) and the widths at every point; the kernels multiply (the results agree to
+// rounding).
+enum RowK { K_RDY, K_RDYF, K_WTH, K_WTHM, K_RDYFM, K_YX, K_XY, K_YZ, K_ZY, K_DLT, K_DLTY, K_DY, K_DYF, K_N };
+
 // The inputs one point reads: every slot on rows j - 1 .. j + 2, loaded into
 // registers before any arithmetic (the reads of the model's branches and of the
-// neighbour rows are then all in flight at once instead of in dependent groups).
-// at() is called with rows j + const, so the window index folds to a constant.
+// neighbour rows are then all in flight at once instead of in dependent groups), and
+// the grid's rows j - 1 .. j + 1 in the model's precision.  at() and rc() are called
+// with rows j + const, so the window index folds to a constant.
 template <typename T>
 struct AmdIn {
-  T (*w)[4];       // the kernel's array (apart from j0, so that it can be split into registers)
-  int j0;          // j - 1
-  int nx;          // from row to row
+  T (*w)[4];         // the kernel's arrays (apart from j0, so that they can be split into registers)
+  const T (*k)[K_N];
+  int j0;            // j - 1
+  int nx;            // from row to row
   __device__ T at(int f, int row, long long) const { return w[f][row - j0]; }
+  __device__ T rc(int row, int c) const { return k[row - j0][c]; }
 };
-// NS slots; rows outside 0..Nyp+1 are clamped (no caller uses such a row's value)
+// rows outside 0..Nyp+1 are clamped (no caller uses such a row's value)
+__device__ __forceinline__ int clamp_row(int row, int last) { return row < 0 ? 0 : (row > last ? last : row); }
+template <typename T>
+__device__ __forceinline__ void load_rows(T (*k)[K_N], const AmdArgs& a, int j) {
+  constexpr int rc[9] = {RC_RDY, RC_RDYF, RC_WTH, RC_WTHM, RC_RDYFM, RC_YX, RC_XY, RC_YZ, RC_ZY};
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    const int row = clamp_row(j - 1 + r, a.g.ny + 1);
+    const double* t = a.rowc + (long long)row * RC_COUNT;
+#pragma unroll
+    for (int c = 0; c < 9; ++c) k[r][c] = T(t[rc[c]]);
+    k[r][K_DLT] = T(a.dlt[row]);
+    k[r][K_DLTY] = T(a.dlt[a.g.ny2 + row]);
+    k[r][K_DY] = T(a.dy[row]);
+    k[r][K_DYF] = T(a.dyf[row]);
+  }
+}
+// NS slots
 template <typename T, int NS>
 __device__ __forceinline__ void load_window(AmdIn<T>& in, const AmdArgs& a, int j, long long q) {
-  const int last = a.g.ny + 1;
-  in.j0 = j - 1;
-  in.nx = a.g.nx;
 #pragma unroll
   for (int s = 0; s < NS; ++s)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      int row = j - 1 + r;
-      row = row < 0 ? 0 : (row > last ? last : row);
-      in.w[s][r] = ((const T*)a.f[s])[(long long)row * a.g.nx + q];
-    }
+    for (int r = 0; r < 4; ++r)
+      in.w[s][r] = ((const T*)a.f[s])[(long long)clamp_row(j - 1 + r, a.g.ny + 1) * a.g.nx + q];
 }
 
-// The reference divides by dy(j), dyf(j) and the filter widths at every point;
-// the row table holds those quotients (RowCoef), so the kernels multiply (the
-// results agree to rounding).
-__device__ __forceinline__ const double* rq(const AmdArgs& a, int j) { return a.rowc + (long long)j * RC_COUNT; }
 // the GY interpolation of GYF values c (row j) and m (row j-1):
 // (c dyf(j-1) + m dyf(j)) / (2 dy(j))
-template <typename R>
-__device__ __forceinline__ R gy_interp(const AmdArgs& a, int j, R c, R m) {
-  const double* rc = rq(a, j);
-  return c * R(rc[RC_WTH]) + m * R(rc[RC_WTHM]);
+template <typename T>
+__device__ __forceinline__ T gy_interp(const AmdIn<T>& in, int j, T c, T m) {
+  return c * in.rc(j, K_WTH) + m * in.rc(j, K_WTHM);
 }
 
 // field slots: 3*f + {0: v, 1: dv/dx, 2: dv/dz}, f = 0 u1, 1 u2, 2 u3, 3+n th_n
@@ -205,7 +222,7 @@ __device__ __forceinline__ Gyf<T> gyf_plane(const AmdIn<T>& in, const AmdArgs& a
   Gyf<T> r;
   const R du1dz = in.at(2, j, q), du3dx = in.at(7, j, q);
   r.a1 = in.at(1, j, q);                                              // SI11 = du1/dx
-  r.a2 = (in.at(3, j + 1, q) - in.at(3, j, q)) * R(rq(a, j)[RC_RDYF]);    // SI22 = du2/dy
+  r.a2 = (in.at(3, j + 1, q) - in.at(3, j, q)) * in.rc(j, K_RDYF);    // SI22 = du2/dy
   r.a3 = in.at(8, j, q);                                              // SI33 = du3/dz
   r.a5 = R(0.5) * (du1dz * R(a.zx) + du3dx * R(a.xz));                // SI13
   r.o5 = R(0.5) * (du1dz * R(a.zx) - du3dx * R(a.xz));                // O13
@@ -216,8 +233,7 @@ __device__ __forceinline__ Gy<T> gy_plane(const AmdIn<T>& in, const AmdArgs& a, 
   using R = T;
   Gy<T> r;
   // the width ratios 2 dy / (dx beta), ... of the scaled gradient, from the row table
-  const double* rc = rq(a, j);
-  const R rdy = R(rc[RC_RDY]), yx = R(rc[RC_YX]), xy = R(rc[RC_XY]), yz = R(rc[RC_YZ]), zy = R(rc[RC_ZY]);
+  const R rdy = in.rc(j, K_RDY), yx = in.rc(j, K_YX), xy = in.rc(j, K_XY), yz = in.rc(j, K_YZ), zy = in.rc(j, K_ZY);
   const R du1dy = (in.at(0, j, q) - in.at(0, j - 1, q)) * rdy;
   const R du3dy = (in.at(6, j, q) - in.at(6, j - 1, q)) * rdy;
   const R du2dx = in.at(4, j, q), du2dz = in.at(5, j, q);
@@ -237,9 +253,9 @@ __device__ __forceinline__ R amd_coef(R a1, R a2, R a3, R a4, R a5, R a6,
              R(6.0) * a4 * a5 * a6;
   v = -v - a1 * (o4 * o4) - a1 * (o5 * o5) - a2 * (o4 * o4) - a2 * (o6 * o6) - a3 * (o5 * o5) -
       a3 * (o6 * o6) - R(2.0) * a4 * o5 * o6 + R(2.0) * a5 * o4 * o6 - R(2.0) * a6 * o4 * o5;
-  if (v <= R(0.0)) return R(0.0);
-  return v / (a1 * a1 + a2 * a2 + a3 * a3 + R(2.0) * (a4 * a4) + R(2.0) * (o4 * o4) + R(2.0) * (a5 * a5) +
-              R(2.0) * (o5 * o5) + R(2.0) * (a6 * a6) + R(2.0) * (o6 * o6));
+  const R d = a1 * a1 + a2 * a2 + a3 * a3 + R(2.0) * (a4 * a4) + R(2.0) * (o4 * o4) + R(2.0) * (a5 * a5) +
+              R(2.0) * (o5 * o5) + R(2.0) * (a6 * a6) + R(2.0) * (o6 * o6);
+  return v <= R(0.0) ? R(0.0) : v / d;
 }
 
 // coefficient at GYF j (GY entries averaged from j and j+1)
@@ -257,7 +273,7 @@ __device__ __forceinline__ T coef_gy(const AmdIn<T>& in, const AmdArgs& a, int j
   using R = T;
   const Gyf<T> f = gyf_plane(in, a, j, q), fm = gyf_plane(in, a, j - 1, q);
   const Gy<T> p = gy_plane(in, a, j, q);
-  auto w = [&](R c, R m) { return gy_interp(a, j, c, m); };
+  auto w = [&](R c, R m) { return gy_interp(in, j, c, m); };
   return amd_coef(w(f.a1, fm.a1), w(f.a2, fm.a2), w(f.a3, fm.a3), p.a4, w(f.a5, fm.a5), p.a6, p.o4,
                   w(f.o5, fm.o5), p.o6);
 }
@@ -276,13 +292,13 @@ template <typename T>
 __device__ __forceinline__ Sgyf<T> sgyf_plane(const AmdIn<T>& in, const AmdArgs& a, int j, long long q) {
   using R = T;
   const R du1dz = in.at(2, j, q), du3dx = in.at(7, j, q);
-  return {in.at(1, j, q), (in.at(3, j + 1, q) - in.at(3, j, q)) * R(rq(a, j)[RC_RDYF]), in.at(8, j, q),
+  return {in.at(1, j, q), (in.at(3, j + 1, q) - in.at(3, j, q)) * in.rc(j, K_RDYF), in.at(8, j, q),
           R(0.5) * (du1dz + du3dx), R(0.5) * (du1dz - du3dx)};
 }
 template <typename T>
 __device__ __forceinline__ Sgy<T> sgy_plane(const AmdIn<T>& in, const AmdArgs& a, int j, long long q) {
   using R = T;
-  const R rdy = R(rq(a, j)[RC_RDY]);
+  const R rdy = in.rc(j, K_RDY);
   const R du1dy = (in.at(0, j, q) - in.at(0, j - 1, q)) * rdy;
   const R du3dy = (in.at(6, j, q) - in.at(6, j - 1, q)) * rdy;
   const R du2dx = in.at(4, j, q), du2dz = in.at(5, j, q);
@@ -302,9 +318,9 @@ __device__ __forceinline__ R amd4_coef(R dX, R dY, R dZ, R a1, R a2, R a3,
   v = -v - dY * a1 * (o4 * o4) - dZ * a1 * (o5 * o5) - dX * a2 * (o4 * o4) - dZ * a2 * (o6 * o6) -
       dX * a3 * (o5 * o5) - dY * a3 * (o6 * o6) - R(2.0) * dZ * a4 * o5 * o6 + R(2.0) * dY * a5 * o4 * o6 -
       R(2.0) * dX * a6 * o4 * o5;
-  if (v <= R(0.0)) return R(0.0);
-  return v / (a1 * a1 + a2 * a2 + a3 * a3 + R(2.0) * (a4 * a4) + R(2.0) * (o4 * o4) + R(2.0) * (a5 * a5) +
-              R(2.0) * (o5 * o5) + R(2.0) * (a6 * a6) + R(2.0) * (o6 * o6));
+  const R d = a1 * a1 + a2 * a2 + a3 * a3 + R(2.0) * (a4 * a4) + R(2.0) * (o4 * o4) + R(2.0) * (a5 * a5) +
+              R(2.0) * (o5 * o5) + R(2.0) * (a6 * a6) + R(2.0) * (o6 * o6);
+  return v <= R(0.0) ? R(0.0) : v / d;
 }
 
 // the model coefficient at GYF j (s1 of les_chan) and at GY j (temp)
@@ -326,7 +342,7 @@ __device__ __forceinline__ T model_gyf(const AmdIn<T>& in, const AmdArgs& a, int
       return sqrt(R(2.0) * (f.s1 * f.s1) + R(4.0) * (s4 * s4) + R(4.0) * (f.s5 * f.s5) + R(2.0) * (f.s2 * f.s2) +
                   R(4.0) * (s6 * s6) + R(2.0) * (f.s3 * f.s3));
     } else {
-      const R dY = (R(a.dy[j]) * R(2.0)) * (R(a.dy[j]) * R(2.0));
+      const R dY = (in.rc(j, K_DY) * R(2.0)) * (in.rc(j, K_DY) * R(2.0));
       return amd4_coef(R(a.dxs) * R(a.dxs), dY, R(a.dzs) * R(a.dzs), f.s1, f.s2, f.s3, s4, f.s5, s6, R(0.5) * (p.o4 + m.o4),
                        f.o5, R(0.5) * (p.o6 + m.o6), false);
     }
@@ -342,13 +358,13 @@ __device__ __forceinline__ T model_gy(const AmdIn<T>& in, const AmdArgs& a, int 
   } else {
     const Sgyf<T> f = sgyf_plane(in, a, j, q), fm = sgyf_plane(in, a, j - 1, q);
     const Sgy<T> p = sgy_plane(in, a, j, q);
-    auto w = [&](R c, R m) { return gy_interp(a, j, c, m); };
+    auto w = [&](R c, R m) { return gy_interp(in, j, c, m); };
     const R s1 = w(f.s1, fm.s1), s2 = w(f.s2, fm.s2), s3 = w(f.s3, fm.s3), s5 = w(f.s5, fm.s5);
     if constexpr (MODEL == 1) {  // (for/les.f90:114-132)
       return sqrt(R(2.0) * (s1 * s1) + R(4.0) * (p.s4 * p.s4) + R(4.0) * (s5 * s5) + R(2.0) * (s2 * s2) + R(4.0) * (p.s6 * p.s6) +
                   R(2.0) * (s3 * s3));
     } else {
-      const R dY = (R(a.dy[j]) * R(2.0)) * (R(a.dy[j]) * R(2.0));
+      const R dY = (in.rc(j, K_DY) * R(2.0)) * (in.rc(j, K_DY) * R(2.0));
       return amd4_coef(R(a.dxs) * R(a.dxs), dY, R(a.dzs) * R(a.dzs), s1, s2, s3, p.s4, s5, p.s6, p.o4, w(f.o5, fm.o5), p.o6,
                        true);
     }
@@ -367,13 +383,12 @@ template <typename T>
 __device__ __forceinline__ ThCoef<T> amd_th_gy(const AmdIn<T>& in, const AmdArgs& a, int ft, int j, long long q) {
   using R = T;
   const R dxs2 = R(a.dxs) * R(a.dxs), dzs2 = R(a.dzs) * R(a.dzs);
-  const R dyl = R(a.dy[j]) * R(2.0), dyl2 = dyl * dyl;
-  const double* rc = rq(a, j);
-  const R rdy = R(rc[RC_RDY]);
-  auto w = [&](int s) { return gy_interp(a, j, in.at(s, j, q), in.at(s, j - 1, q)); };
+  const R dyl = in.rc(j, K_DY) * R(2.0), dyl2 = dyl * dyl;
+  const R rdy = in.rc(j, K_RDY);
+  auto w = [&](int s) { return gy_interp(in, j, in.at(s, j, q), in.at(s, j - 1, q)); };
   const R du1dx = w(1), du3dz = w(8), du1dz = w(2), du3dx = w(7);
-  const R du2dy = gy_interp(a, j, (in.at(3, j + 1, q) - in.at(3, j, q)) * R(rc[RC_RDYF]),
-                            (in.at(3, j, q) - in.at(3, j - 1, q)) * R(rc[RC_RDYFM]));
+  const R du2dy = gy_interp(in, j, (in.at(3, j + 1, q) - in.at(3, j, q)) * in.rc(j, K_RDYF),
+                            (in.at(3, j, q) - in.at(3, j - 1, q)) * in.rc(j, K_RDYFM));
   const R tx = w(ft + 1), tz = w(ft + 2);
   const R ty = (in.at(ft, j, q) - in.at(ft, j - 1, q)) * rdy;
   const R du1dy = (in.at(0, j, q) - in.at(0, j - 1, q)) * rdy;
@@ -390,12 +405,12 @@ template <typename T>
 __device__ __forceinline__ ThCoef<T> amd_th_gyf(const AmdIn<T>& in, const AmdArgs& a, int ft, int j, long long q) {
   using R = T;
   const R dxs2 = R(a.dxs) * R(a.dxs), dzs2 = R(a.dzs) * R(a.dzs);
-  const R dyl = R(a.dyf[j]) * R(2.0), dyl2 = dyl * dyl;
-  auto gyv = [&](int s, int jj) { return (in.at(s, jj, q) - in.at(s, jj - 1, q)) * R(rq(a, jj)[RC_RDY]); };
+  const R dyl = in.rc(j, K_DYF) * R(2.0), dyl2 = dyl * dyl;
+  auto gyv = [&](int s, int jj) { return (in.at(s, jj, q) - in.at(s, jj - 1, q)) * in.rc(jj, K_RDY); };
   const R tx = in.at(ft + 1, j, q), tz = in.at(ft + 2, j, q);
   const R ty = R(0.5) * (gyv(ft, j + 1) + gyv(ft, j));
   const R du1dx = in.at(1, j, q), du3dz = in.at(8, j, q);
-  const R du2dy = (in.at(3, j + 1, q) - in.at(3, j, q)) * R(rq(a, j)[RC_RDYF]);
+  const R du2dy = (in.at(3, j + 1, q) - in.at(3, j, q)) * in.rc(j, K_RDYF);
   const R du1dy = R(0.5) * (gyv(0, j + 1) + gyv(0, j)), du3dy = R(0.5) * (gyv(6, j + 1) + gyv(6, j));
   const R du2dx = R(0.5) * (in.at(4, j + 1, q) + in.at(4, j, q));
   const R du2dz = R(0.5) * (in.at(5, j + 1, q) + in.at(5, j, q));
@@ -412,17 +427,17 @@ __device__ __forceinline__ ThCoef<T> amd_th_gyf(const AmdIn<T>& in, const AmdArg
 // at j = 2, for/les.f90:454, 762), type 1 multiplies it (for/les.f90:145); that
 // row feeds only rows the BC rows overwrite.
 // coef: model_gy at row j (unused on the row-1 special case).
-template <int MODEL, typename T>
+template <int MODEL, bool INNER, typename T>
 __device__ __forceinline__ T tau_gy(const AmdIn<T>& in, const AmdArgs& a, int e, int j, long long q, T coef) {
   using R = T;
-  const R dlt = R(a.dlt[a.g.ny2 + j]);
+  const R dlt = in.rc(j, K_DLTY);
   const R half = R(0.5) * in.at(e ? 5 : 4, j, q);
-  if constexpr (MODEL == 1) return dlt * (coef * half);
+  if constexpr (MODEL == 1 || INNER) return dlt * (coef * half);
   // the row asked for through a copy of j: where the compiler knows that j is 1 it
   // addresses the window by 2 - j, in memory
   int jc = j;
   asm("" : "+s"(jc));
-  const R dvdy = (in.at(e ? 6 : 0, j, q) - in.at(e ? 6 : 0, j - 1, q)) * R(rq(a, j)[RC_RDY]);
+  const R dvdy = (in.at(e ? 6 : 0, j, q) - in.at(e ? 6 : 0, j - 1, q)) * in.rc(j, K_RDY);
   return jc == 1 ? dlt * R(0.5) * (dvdy + in.at(e ? 5 : 4, j, q)) : dlt * (coef * half);
 }
 
@@ -443,12 +458,13 @@ __device__ __forceinline__ void xcd_rows(int b, int nqb, int nj, int& qb, int& j
 }
 
 // The model at one point of row j: nu_t and kappa_t (GY), and the additions to the
-// products.
+// products.  INNER: a row on which every term is present (les_inner), without the
+// tests, so that the strains three coefficients share are formed once.
 template <typename T, int NTH>
 struct AmdOut {
   T nut, kap[NTH > 0 ? NTH : 1], A[7 + 2 * NTH];
 };
-template <typename T, int NTH, int MODEL>
+template <typename T, int NTH, int MODEL, bool INNER>
 __device__ __forceinline__ void amd_point(const AmdIn<T>& in, const AmdArgs& a, int j, long long q, AmdOut<T, NTH>& r) {
   using R = T;
   const Geo& g = a.g;
@@ -457,36 +473,35 @@ __device__ __forceinline__ void amd_point(const AmdIn<T>& in, const AmdArgs& a, 
   // the model coefficient at GY j and j + 1, each evaluated once: nu_t, the two
   // stresses at GY j and the GYF flux differences take them (row 1 of types 4
   // and 5 needs none)
-  const bool need_j = j <= ny && (j >= 2 || (MODEL == 1 && j == 1));
+  const bool need_j = INNER || (j <= ny && (j >= 2 || (MODEL == 1 && j == 1)));
   const R cj = need_j ? model_gy<MODEL>(in, a, j, q) : R(0.0);
-  const R cj1 = (j >= a.jstart && j <= ny - 1) ? model_gy<MODEL>(in, a, j + 1, q) : R(0.0);
-  const double* rc = rq(a, j);
+  const R cj1 = (INNER || (j >= a.jstart && j <= ny - 1)) ? model_gy<MODEL>(in, a, j + 1, q) : R(0.0);
   // nu_t at GY j (zero on the wall rows of ghost_les_mpi)
   r.nut = R(0.0);
-  if (j >= 3 && j <= ny - 1) r.nut = -R(0.5) * R(a.dlt[g.ny2 + j]) * cj;
+  if (INNER || (j >= 3 && j <= ny - 1)) r.nut = -R(0.5) * in.rc(j, K_DLTY) * cj;
 #pragma unroll
   for (int m = 0; m < 7 + 2 * NTH; ++m) r.A[m] = R(0.0);
   // GYF stresses, rows j1..j2 = jstart..Nyp-1
-  if (j >= a.jstart && j <= ny - 1) {
-    const R dyf = R(a.dlt[j]) * model_gyf<MODEL>(in, a, j, q);
+  if (INNER || (j >= a.jstart && j <= ny - 1)) {
+    const R dyf = in.rc(j, K_DLT) * model_gyf<MODEL>(in, a, j, q);
     const R du1dz = in.at(2, j, q), du3dx = in.at(7, j, q);
     r.A[0] = dyf * in.at(1, j, q);
     r.A[1] = dyf * (R(0.5) * (du1dz + du3dx));
     r.A[2] = dyf * in.at(8, j, q);
-    const R rdyf = R(rc[RC_RDYF]);
-    r.A[3] = (tau_gy<MODEL>(in, a, 0, j + 1, q, cj1) - tau_gy<MODEL>(in, a, 0, j, q, cj)) * rdyf;
-    r.A[4] = (tau_gy<MODEL>(in, a, 1, j + 1, q, cj1) - tau_gy<MODEL>(in, a, 1, j, q, cj)) * rdyf;
+    const R rdyf = in.rc(j, K_RDYF);
+    r.A[3] = (tau_gy<MODEL, INNER>(in, a, 0, j + 1, q, cj1) - tau_gy<MODEL, INNER>(in, a, 0, j, q, cj)) * rdyf;
+    r.A[4] = (tau_gy<MODEL, INNER>(in, a, 1, j + 1, q, cj1) - tau_gy<MODEL, INNER>(in, a, 1, j, q, cj)) * rdyf;
   }
   // GY stresses and the explicit cross terms, rows 2..Nyp
-  if (j >= 2 && j <= ny) {
-    const R rdy = R(rc[RC_RDY]);
-    r.A[5] = tau_gy<MODEL>(in, a, 0, j, q, cj) - r.nut * ((in.at(0, j, q) - in.at(0, j - 1, q)) * rdy);
-    r.A[6] = tau_gy<MODEL>(in, a, 1, j, q, cj) - r.nut * ((in.at(6, j, q) - in.at(6, j - 1, q)) * rdy);
+  if (INNER || (j >= 2 && j <= ny)) {
+    const R rdy = in.rc(j, K_RDY);
+    r.A[5] = tau_gy<MODEL, INNER>(in, a, 0, j, q, cj) - r.nut * ((in.at(0, j, q) - in.at(0, j - 1, q)) * rdy);
+    r.A[6] = tau_gy<MODEL, INNER>(in, a, 1, j, q, cj) - r.nut * ((in.at(6, j, q) - in.at(6, j - 1, q)) * rdy);
   }
 #pragma unroll
   for (int n = 0; n < NTH; ++n) {
     const int ft = 3 * (3 + n);
-    const bool row = (j >= a.jstart_th[n] && j <= a.jend_th[n]);
+    const bool row = INNER || (j >= a.jstart_th[n] && j <= a.jend_th[n]);
     r.kap[n] = R(0.0);
     if constexpr (MODEL == 1 || MODEL == 4) {
       // les_chan_th types 1 and 4 (for/les.f90:1118-1193): kappa_t = nu_t (GY), and
@@ -497,11 +512,11 @@ __device__ __forceinline__ void amd_point(const AmdIn<T>& in, const AmdArgs& a, 
     } else {
       // les_chan_th type 5; type 6 reads the learned coefficients.
       // kappa_t at GY j (for/les.f90:1259-1306, 1344-1348)
-      if (j >= 3 && j <= ny - 1) {
+      if (INNER || (j >= 3 && j <= ny - 1)) {
         R c;
         if constexpr (MODEL == 6) c = fabs((R)((const T*)a.kgy)[o]);
         else c = amd_th_gy(in, a, ft, j, q).c;
-        r.kap[n] = -R(0.5) * R(a.dlt[g.ny2 + j]) * c;
+        r.kap[n] = -R(0.5) * in.rc(j, K_DLTY) * c;
       }
       // SGS flux at GYF j (for/les.f90:1221-1256, 1310-1318, 1372-1393)
       if (row) {
@@ -512,7 +527,7 @@ __device__ __forceinline__ void amd_point(const AmdIn<T>& in, const AmdArgs& a, 
         } else {
           s1 = amd_th_gyf(in, a, ft, j, q).c;
         }
-        const R f = R(0.5) * R(a.dlt[j]) * s1;
+        const R f = R(0.5) * in.rc(j, K_DLT) * s1;
         r.A[7 + 2 * n] = f * in.at(ft + 1, j, q);
         r.A[8 + 2 * n] = f * in.at(ft + 2, j, q);
       }
@@ -520,8 +535,19 @@ __device__ __forceinline__ void amd_point(const AmdIn<T>& in, const AmdArgs& a, 
   }
 }
 
+// whether row j has every term of amd_point and les_products (all rows but those at
+// the walls)
+template <int NTH>
+__device__ __forceinline__ bool les_inner(const XProdArgs& x, const AmdArgs& a, int j) {
+  bool in = j >= 3 && j >= a.jstart && j >= x.jstart && j <= a.g.ny - 1 && j <= x.jend;
+#pragma unroll
+  for (int n = 0; n < NTH; ++n)
+    in = in && j >= a.jstart_th[n] && j <= a.jend_th[n] && j >= x.jstart_th[n] && j <= x.jend_th[n];
+  return in;
+}
+
 // The products of xprod_products at one point, plus the SGS additions.
-template <typename T, int NTH>
+template <typename T, int NTH, bool INNER>
 __device__ __forceinline__ void les_products(const XProdArgs& x, const AmdIn<T>& in, int j, const AmdOut<T, NTH>& r,
                                              T* P) {
   const int ny = x.g.ny;
@@ -529,20 +555,19 @@ __device__ __forceinline__ void les_products(const XProdArgs& x, const AmdIn<T>&
   const T u0 = in.w[0][0], u = in.w[0][1], up = in.w[0][2];
   const T v0 = in.w[3][0], v = in.w[3][1], vp = in.w[3][2];
   const T w0 = in.w[6][0], w = in.w[6][1], wp = in.w[6][2];
-  const double* rc = x.rowc + (long long)j * RC_COUNT;
-  const T rdy = (T)rc[RC_RDY], r2f = T(0.5) * (T)rc[RC_RDYF];
-  const T dyfj = (T)x.dyf[j], dyfm = (T)x.dyf[j - 1];
+  const T rdy = in.rc(j, K_RDY), r2f = T(0.5) * in.rc(j, K_RDYF);
+  const T dyfj = in.rc(j, K_DYF), dyfm = in.rc(j - 1, K_DYF);
   const T cint = T(0.5) * rdy;
 #pragma unroll
   for (int p = 0; p < 8 + 3 * NTH; ++p) P[p] = T(0);
-  if (j >= x.jstart && j <= x.jend) {
+  if (INNER || (j >= x.jstart && j <= x.jend)) {
     P[0] = w * u + r.A[1];
     P[1] = u * u + r.A[0];
     P[2] = w * w + r.A[2];
     P[5] = (up * vp + u * vp - u * v - u0 * v) * r2f + r.A[3];
     P[6] = (wp * vp + w * vp - w * v - w0 * v) * r2f + r.A[4];
   }
-  if (j >= 2 && j <= ny) {
+  if (INNER || (j >= 2 && j <= ny)) {
     P[3] = ((dyfj * u + dyfm * u0) * cint) * v + r.A[5];
     P[4] = ((dyfj * w + dyfm * w0) * cint) * v + r.A[6];
     const T ap = v + vp, am = v + v0;
@@ -551,12 +576,21 @@ __device__ __forceinline__ void les_products(const XProdArgs& x, const AmdIn<T>&
 #pragma unroll
   for (int n = 0; n < NTH; ++n) {
     const T t0 = in.w[9 + 3 * n][0], t = in.w[9 + 3 * n][1], tp = in.w[9 + 3 * n][2];
-    if (j >= x.jstart_th[n] && j <= x.jend_th[n]) {
+    if (INNER || (j >= x.jstart_th[n] && j <= x.jend_th[n])) {
       P[8 + 3 * n] = t * u + r.A[7 + 2 * n];
       P[9 + 3 * n] = t * w + r.A[8 + 2 * n];
       P[10 + 3 * n] = (tp * vp + t * vp - t * v - t0 * v) * r2f;
     }
   }
+}
+
+// b in scalar registers and opaque.  In float the bases are formed one after another
+// (volatile): all at once they spill to memory with two scalars.  In FP64 the order
+// costs registers the other way (one block per CU at 512 lines).
+template <typename T>
+__device__ __forceinline__ void scalar_base(const char*& b) {
+  if constexpr (sizeof(T) == 4) asm volatile("" : "+s"(b));
+  else asm("" : "+s"(b));
 }
 
 // SPLIT: the order of the product lines, u1's and u3's equations (u1u1, flux of u1,
@@ -615,11 +649,21 @@ __device__ __forceinline__ void les_store(const cx<T>* __restrict__ s, const Geo
 // and two or more blocks share a CU (where the whole tile leaves room for one, a
 // CU's loads, arithmetic and transforms run one after another).
 //
+// The model takes more instructions than the transforms, so a point's are kept down:
+// the rows' grid quotients are read and converted once per block, addresses are a
+// scalar base and 32 bits per lane, and rows away from the walls run without tests
+// (with all three in the point's code: 4370 us FP64, 2080 float).  512 threads per
+// block in float, 4 waves per SIMD instead of 3: 1846 against 1825 us.
+//
 // One launch, against the model and product kernels it replaces: 512x257x512 FP64
-// 6350 -> 4240 us (in one piece: 5505), float 2796 -> 2070; 128x129x128 FP64
-// (in one piece) 213 -> 115.
+// 6350 -> 3220 us, float 2796 -> 1825; 128x129x128 FP64 (in one piece) 213 -> 116.
+// (two blocks of 256 threads, where LDS has room for them, leave 256 registers each)
+template <typename T, int NX, int NTH, bool SPLIT>
+constexpr int les_waves() {
+  return SPLIT && 2 * sizeof(cx<T>) * (NTH == 2 ? 10 : 6 + NTH) * NX <= 163840 ? 2 : 1;
+}
 template <typename T, int NX, int NT, int NTH, int MODEL, bool SPLIT>
-__global__ __launch_bounds__(NT) void k_les_products(XProdArgs x, AmdArgs a, int nj) {
+__global__ __launch_bounds__(NT, (les_waves<T, NX, NTH, SPLIT>())) void k_les_products(XProdArgs x, AmdArgs a, int nj) {
   constexpr int NP = 8 + 3 * NTH, NA = 5, NB = NP - NA;
   constexpr int NL = SPLIT ? (NA > NB ? NA : NB) : NP;
   constexpr int K = (2 * NX + NT - 1) / NT;  // points per thread
@@ -634,21 +678,51 @@ __global__ __launch_bounds__(NT) void k_les_products(XProdArgs x, AmdArgs a, int
   // one value to the compiler: the window's row differences fold to constants
   const int j = __builtin_amdgcn_readfirstlane(x.jlo + jj);
   T PB[SPLIT ? K : 1][NB];
-  // point c of the pair: line c / NX, column c mod NX
-  auto point = [&](int c, T* pb) __attribute__((always_inline)) {
-    const int xc = c & (NX - 1), line = c / NX;
-    const long long q = pcol(g, (long long)(z + line) * NX + xc), o = (long long)j * NX + q;
+  T rows[3][K_N];
+  load_rows<T>(rows, a, j);
+  // Point k of the thread: column xc of line `line`, c = tid + k NT = line NX + xc.  The
+  // plane's first column is the same for the block, and the line too where a line is
+  // NT points or more, so that base addresses are scalar and a lane adds 32 bits.
+  auto point = [&](auto inner, int k, T* pb) __attribute__((always_inline)) {
+    constexpr bool INNER = decltype(inner)::value;
+    const int kl = NX >= NT ? k * NT / NX : 0;  // line, the lane's part of it
+    const int c = NX >= NT ? tid + k * NT % NX : tid;
+    const int xc = c & (NX - 1), ll = NX >= NT ? 0 : c / NX, line = kl + ll;
+    unsigned lane = (unsigned)(ll * g.ny2 * NX + xc) * (unsigned)sizeof(T);
+    asm("" : "+v"(lane));  // formed here: a 64-bit copy made before the loop would be added to each base
+    const long long q = (long long)(z + kl) * g.ny2 * NX;  // lane apart
+    auto addr = [&](const void* f, int row) { return (const char*)f + (q + (long long)row * NX) * (long long)sizeof(T); };
     T win[3 * (3 + NTH)][4];
     AmdIn<T> in;
     in.w = win;
-    load_window<T, 3 * (3 + NTH)>(in, a, j, q);
-    AmdOut<T, NTH> r;
-    amd_point<T, NTH, MODEL>(in, a, j, q, r);
-    ((T*)a.nut)[o] = r.nut;
+    in.k = rows;
+    in.j0 = j - 1;
+    in.nx = NX;
+    // one scalar base for the rows a load's immediate offset (+-4 KiB) reaches
+    constexpr int RB = NX * (int)sizeof(T), G = 2 * RB <= 4096 ? 4 : (RB <= 4096 ? 2 : 1);
 #pragma unroll
-    for (int n = 0; n < NTH; ++n) ((T*)a.kap[n])[o] = r.kap[n];
+    for (int f = 0; f < 3 * (3 + NTH); ++f)
+#pragma unroll
+      for (int r0 = 0; r0 < 4; r0 += INNER ? G : 1) {
+        const char* b = addr(a.f[f], INNER ? j - 1 + r0 + G / 2 : clamp_row(j - 1 + r0, g.ny + 1));
+        scalar_base<T>(b);
+#pragma unroll
+        for (int r = 0; r < (INNER ? G : 1); ++r)
+          win[f][r0 + r] =
+              *(const __attribute__((address_space(1))) T*)(b + (INNER ? (r - G / 2) * RB : 0) + lane);
+      }
+    AmdOut<T, NTH> r;
+    amd_point<T, NTH, MODEL, INNER>(in, a, j, q + lane / (unsigned)sizeof(T), r);
+    auto out = [&](void* f, T v) { 
+      const char* b = addr(f, j);
+      scalar_base<T>(b);
+      *(__attribute__((address_space(1))) T*)((char*)b + lane) = v;
+    };
+    out(a.nut, r.nut);
+#pragma unroll
+    for (int n = 0; n < NTH; ++n) out(a.kap[n], r.kap[n]);
     T P[NP];
-    les_products<T, NTH>(x, in, j, r, P);
+    les_products<T, NTH, INNER>(x, in, j, r, P);
     auto put = [&](int slot, T v) { ((T*)&s[slot * NX + swz<T>(xc)])[line] = v; };
     if constexpr (SPLIT) {
 #pragma unroll
@@ -660,13 +734,22 @@ __global__ __launch_bounds__(NT) void k_les_products(XProdArgs x, AmdArgs a, int
       for (int p = 0; p < NP; ++p) put(p, P[p]);
     }
   };
-  if constexpr (SPLIT) {
-    static_assert(2 * NX == K * NT, "whole points");
+  auto points = [&](auto inner) __attribute__((always_inline)) {
+    if constexpr (SPLIT) {
+      static_assert(2 * NX == K * NT, "whole points");
 #pragma unroll
-    for (int k = 0; k < K; ++k) point(tid + k * NT, PB[k]);
-  } else {
-    for (int c = tid; c < 2 * NX; c += NT) point(c, PB[0]);
-  }
+      for (int k = 0; k < K; ++k) point(inner, k, PB[k]);
+    } else {
+#pragma unroll 1
+      for (int k = 0; k < K; ++k)
+        if (2 * NX >= NT || tid < 2 * NX) point(inner, k, PB[0]);
+    }
+  };
+  // (two scalars in halves hold 9 lines of every point in registers: there the rows
+  // without tests spill, 417 us against 342 at 512x65x128 FP64;
+  // the constant-coefficient model does not)
+  if (!(SPLIT && NTH == 2 && MODEL != 1) && les_inner<NTH>(x, a, j)) points(std::true_type{});
+  else points(std::false_type{});
   __syncthreads();
   if constexpr (SPLIT) {
     fft_lds_sync<T, NX, NA, NT, -1>(s, NX, stw, tid);

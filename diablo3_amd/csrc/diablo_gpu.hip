@@ -574,8 +574,9 @@ int launch_les_products(dgpu_handle* h, XProdArgs& x, const AmdArgs& a, int nj) 
       return fail(2, "this nx needs the mixed-precision mode (x pass exceeds LDS in FP64)");
     } else {
       // the tile in two halves where the whole one (> 80 KiB) leaves room for one
-      // block per CU only (512 lines FP64: 5505 us in one piece, 4240 in two); below,
-      // two or more blocks fit as it is and the halves only add barriers
+      // block per CU only (512 lines FP64, before the model's code was cut down: 5505 us
+      // in one piece, 4240 in two); below, two or more blocks fit as it is and the
+      // halves only add barriers
       constexpr int NT = les_nt(N_);
       k_les_products<T, N_, NT, NTH, MODEL, (lds > 81920)>
           <<<(unsigned)(h->g.nz / 2 * nj), NT, 0, h->st>>>(x, a, nj);
