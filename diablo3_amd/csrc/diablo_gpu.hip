@@ -68,6 +68,14 @@ constexpr int ti_for(int nz, int sz) {
   int t = 32768 / (nz * sz);
   return t < 2 ? 2 : (t > 16 ? 16 : t);
 }
+// Columns and threads of a k_inv_z / k_fwd_z block.  LDS lets four 32 KiB tiles share
+// a CU: from 256 points a float tile has work for 512 threads, whose registers fit 8
+// waves per SIMD (512 points, 257 planes: v and dv/dz 815 -> 656 us, increments' forward 618 ->
+// 539; 256 points: 59 -> 48).  In FP64 512 threads take registers that leave 5 waves
+// (59 -> 65 us at 256 points), but at 512 points two tiles of 8 columns, whose rows fill
+// a 128-byte line, do better than four of 4 (1087 -> 912, forward 696 -> 606 us).
+constexpr int z_cols(int nz, int sz) { return nz == 512 && sz == 16 ? 8 : ti_for(nz, sz); }
+constexpr int z_nt(int nz, int sz) { return (sz == 8 ? nz >= 256 : nz == 512) ? 512 : 256; }
 
 }  // namespace
 
@@ -157,9 +165,9 @@ struct dgpu_handle {
   long long t_n[16] = {};
 };
 
-// Transform scratch of dgpu_fft_xz_to_fourier_noalloc: the compact physical field,
-// the x-spectra and the packed spectrum of one grid, in one file-scope device
-// array (each GPU the library runs on holds its own copy until the process
+// Transform scratch of dgpu_fft_xz_to_fourier_noalloc (the x-spectra of one grid,
+// with room for the compact physical field and the packed spectrum, which the
+// interface's size bound counts), in one file-scope device array (each GPU the library runs on holds its own copy until the process
 // ends).  Host code never passes `scratch` itself to a kernel: its per-device
 // address comes from hipGetSymbolAddress at dgpu_create.
 constexpr size_t kNoallocScratchBytes = (size_t)DGPU_NOALLOC_SCRATCH_BYTES;
@@ -484,9 +492,9 @@ int launch_inv_z(dgpu_handle* h, int nf, const cd* const* src, void* const* dst,
   for (int f = 0; f < nf; ++f) { s.p[f] = src[f]; d.p[f] = (cx<T>*)dst[f]; }
   const cx<T>* tw = (const cx<T>*)(sizeof(T) == 8 ? h->twz64 : h->twz32);
   DG_SWITCH_N(h->g.nz, {
-    constexpr int TI = ti_for(N_, sizeof(cx<T>));
+    constexpr int TI = z_cols(N_, sizeof(cx<T>)), NT = z_nt(N_, sizeof(cx<T>));
     const int grid = batch_grid((h->g.kxr + TI - 1) / TI * nj, nf, ZK<T, TI>);
-    k_inv_z<T, N_, TI, 256><<<grid, 256, 0, h->st>>>(s, d, h->g, j0, nj, nf, tw, h->d_kz, dzmask);
+    k_inv_z<T, N_, TI, NT><<<grid, NT, 0, h->st>>>(s, d, h->g, j0, nj, nf, tw, h->d_kz, dzmask);
   });
   HIPCHK(hipGetLastError());
   return 0;
@@ -502,9 +510,9 @@ int launch_fwd_z(dgpu_handle* h, int nf, void* const* src, cd* const* dst, int j
   for (int f = 0; f < nf; ++f) { s.p[f] = (const cx<T>*)src[f]; d.p[f] = dst[f]; }
   const cx<T>* tw = (const cx<T>*)(sizeof(T) == 8 ? h->twz64 : h->twz32);
   DG_SWITCH_N(h->g.nz, {
-    constexpr int TI = ti_for(N_, sizeof(cx<T>));
+    constexpr int TI = z_cols(N_, sizeof(cx<T>)), NT = z_nt(N_, sizeof(cx<T>));
     dim3 grid((h->g.kxr + TI - 1) / TI, nj, nf);
-    k_fwd_z<T, N_, TI, 256, ACC><<<grid, 256, 0, h->st>>>(s, d, h->g, j0, tw, dj, dk, izero);
+    k_fwd_z<T, N_, TI, NT, ACC><<<grid, NT, 0, h->st>>>(s, d, h->g, j0, tw, dj, dk, izero);
   });
   HIPCHK(hipGetLastError());
   return 0;
@@ -622,30 +630,25 @@ template <typename T>
 int launch_fwdz_nl(dgpu_handle* h, NlArgs& a, int nj) {
   a.tw = sizeof(T) == 8 ? h->twz64 : h->twz32;
   DG_SWITCH_N(h->g.nz, {
-    constexpr int TI0 = ti_for(N_, sizeof(cx<T>));
-    auto go = [&](auto TIc, auto Pc) {
-      constexpr int TI = decltype(TIc)::value;
-      constexpr bool PERSIST = decltype(Pc)::value;
-      const int ntiles = (h->g.kxr + TI - 1) / TI * nj * (3 + h->nth);
-      // persistent: as many blocks as are resident at once (one per CU for the FP64
-      // 72 KiB tile at nz = 256: 0.126 -> 0.118 ms against two per CU)
-      if (PERSIST && h->fz_resident <= 0) {
-        int per_cu = 0;
-        HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_fwdz_nl<T, N_, TI, 256, PERSIST>, 256, 0));
-        h->fz_resident = std::max(1, per_cu) * h->cus;
-      }
-      const int nblk = PERSIST ? std::min(ntiles, h->fz_resident) : ntiles;
-      k_fwdz_nl<T, N_, TI, 256, PERSIST><<<nblk, 256, 0, h->st>>>(a, ntiles);
-      return 0;
-    };
-    using I0 = std::integral_constant<int, TI0>;
-    using I1 = std::integral_constant<int, (TI0 > 1 ? TI0 / 2 : 1)>;
-    using P0 = std::false_type;
-    using P1 = std::true_type;
-    // measured: FP64 best persistent with TI columns; float with TI/2 per block at
-    // nz = 256 (256^3), persistent with TI columns at nz = 512 (512x257x512)
-    const int rc = (sizeof(T) == 8 || h->g.nz >= 512) ? go(I0{}, P1{}) : go(I1{}, P0{});
-    if (rc) return rc;
+    // FP64: one tile (2 x 32 KiB) per block at 256 and 512 points, where two blocks
+    // share a CU (512 points, 257 planes: 872 us against 996 persistent; 256: 108
+    // against 115); persistent at 1024, where one has it to itself (62 us against 76,
+    // 33 planes), and below (128: 32.2 against 32.6).  Float: persistent with 512 threads
+    // from 512 points (630 us; 256 threads 748, one tile per block 767), half the
+    // columns and one tile per block below (256 points: 56 us, persistent 69).
+    constexpr bool F = sizeof(T) == 4;
+    constexpr bool PERSIST = F ? N_ >= 512 : N_ != 256 && N_ != 512;
+    constexpr int NT = F && N_ >= 512 ? 512 : 256;
+    constexpr int TI0 = ti_for(N_, sizeof(cx<T>)), TI = F && N_ < 512 ? TI0 / 2 : TI0;
+    const int ntiles = (h->g.kxr + TI - 1) / TI * nj * (3 + h->nth);
+    // persistent: as many blocks as are resident at once
+    if (PERSIST && h->fz_resident <= 0) {
+      int per_cu = 0;
+      HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_fwdz_nl<T, N_, TI, NT, PERSIST>, NT, 0));
+      h->fz_resident = std::max(1, per_cu) * h->cus;
+    }
+    const int nblk = PERSIST ? std::min(ntiles, h->fz_resident) : ntiles;
+    k_fwdz_nl<T, N_, TI, NT, PERSIST><<<nblk, NT, 0, h->st>>>(a, ntiles);
   });
   HIPCHK(hipGetLastError());
   return 0;
