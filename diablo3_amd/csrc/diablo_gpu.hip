@@ -165,10 +165,10 @@ struct dgpu_handle {
   long long t_n[16] = {};
 };
 
-// Transform scratch of dgpu_fft_xz_to_fourier_noalloc (the x-spectra of one grid,
-// with room for the compact physical field and the packed spectrum, which the
-// interface's size bound counts), in one file-scope device array (each GPU the library runs on holds its own copy until the process
-// ends).  Host code never passes `scratch` itself to a kernel: its per-device
+// Transform scratch of dgpu_fft_xz_to_fourier_noalloc: the x-spectra of one grid (the
+// interface's size limit counts the field and the packed spectrum too), in one
+// file-scope device array; each GPU the library runs on holds its own copy until the
+// process ends.  Host code never passes `scratch` itself to a kernel: its per-device
 // address comes from hipGetSymbolAddress at dgpu_create.
 constexpr size_t kNoallocScratchBytes = (size_t)DGPU_NOALLOC_SCRATCH_BYTES;
 static __device__ __align__(256) unsigned char scratch[kNoallocScratchBytes];
@@ -2121,12 +2121,12 @@ int dgpu_fft_xz_to_fourier_noalloc(dgpu_handle* h, const double* phys, double* f
   const size_t hb = round256(sizeof(cd) * g.ph * g.ny2);
   const size_t cb = round256(sizeof(cd) * g.pc * g.ny2);
   if (rb + hb + cb > kNoallocScratchBytes)
-    return fail(2, "dgpu_fft_xz_to_fourier_noalloc: this grid needs " + std::to_string(rb + hb + cb) +
-                       " bytes of transform scratch; the allocation-free entry point holds " +
+    return fail(2, "dgpu_fft_xz_to_fourier_noalloc: grid too large: field, x-spectra and spectrum take " +
+                       std::to_string(rb + hb + cb) + " bytes, the limit (the size of the static scratch) is " +
                        std::to_string(kNoallocScratchBytes));
-  // the transforms read and write the Fortran arrays themselves (the scratch bound
-  // above is the interface's); the x-spectra are complete before four is written,
-  // so the two may alias
+  // the transforms read and write the Fortran arrays themselves: only the x-spectra
+  // use the scratch (at rb, within the size that the limit allows); they are complete
+  // before four is written, so phys and four may alias
   const double* rs[1] = {phys};
   void* hs[1] = {h->noalloc + rb};
   cd* cs[1] = {(cd*)four};

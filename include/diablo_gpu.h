@@ -155,12 +155,12 @@ int dgpu_fft_xz_to_physical(dgpu_handle *h, const double *four, double *phys);
  * harnesses that forbid hipMalloc).  The same transform, with phys and four in
  * the same Fortran layouts but in DEVICE memory (they may alias, as the
  * reference's u/cu views do); rows k >= 2 Nkz + 1 of four are left untouched.
- * It calls no hipMalloc or hipFree: the compact field, the x-spectra and the
- * packed spectrum live in a library-static device buffer of
- * DGPU_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends, and grids
- * needing more (8 Nx Nz (Ny+2) + 16 kxp (Nz + 2 Nkz + 1)(Ny+2) bytes, kxp = Nkx + 1
- * rounded up to a multiple of 8; 128x129x128 needs 38.6 MB) are rejected with
- * status 2.  The device current at the call must be the handle's.  Every call
+ * It calls no hipMalloc or hipFree: the x-spectra between the two transforms live in
+ * a library-static device buffer of DGPU_NOALLOC_SCRATCH_BYTES per GPU, held until
+ * the process ends.  A limit of the interface: grids whose field, x-spectra and packed
+ * spectrum together (8 Nx Nz (Ny+2), 16 kxp Nz (Ny+2) and 16 kxp (2 Nkz + 1)(Ny+2)
+ * bytes, kxp = Nkx + 1 rounded up to a multiple of 8, each rounded up to 256) exceed
+ * that size are rejected with status 2 (128x129x128: 38.6 MB; 128x226x128: above).  The device current at the call must be the handle's.  Every call
  * on one GPU shares that buffer: calls that overlap on one GPU (two threads,
  * or two handles' streams) race. */
 enum { DGPU_NOALLOC_SCRATCH_BYTES = 64 << 20 };
