@@ -50,11 +50,12 @@ def kernel_bytes(cfg, mixed):
         # product spectra of planes jlo..ny out (physical fields stay on chip)
         "k_xmarch": nf * cfg.kxr * cfg.nz * 2 * s * (nj + 2) + no * Hj,
         "k_fwdz_nl": no * Hj + nf * Cj_t,
-        # nonlinear terms, state, cp and (rk 2, 3: 2 of 3 launches) old cf in; cf and state out
+        # assembly and solves: nonlinear terms, state, cp and (rk 2, 3: 2 of 3 launches)
+        # old cf in; cf and state out
         "k_cn": nf * Cj_t + (nf + 1) * C + (2.0 / 3.0) * nf * Cj + nf * Cj + nf * C,
         "k_project": 4 * C + 4 * C,
     }
-    # DNS: the same with the projection in the kernel: the pressure goes out too
+    # the DNS column pass: the projection too, so that the pressure goes out
     out["k_column"] = out["k_cn"] + C
     if cfg.use_les:
         # physical fields: R8 FP64, Rt in the transform precision
@@ -71,7 +72,7 @@ def kernel_bytes(cfg, mixed):
         if learned:
             out["k_closure"] = 3 * nf * Rt + 4 * Rt
         # assembly only: the right-hand side goes out instead of the solve
-        out["k_cn"] = nf * Cj_t + (nf + 1) * C + (2.0 / 3.0) * nf * Cj + nf * Cj + nf * C
+        out["k_assemble"] = nf * Cj_t + (nf + 1) * C + (2.0 / 3.0) * nf * Cj + nf * Cj + nf * C
         npts = cfg.nx * cfg.nz * ny2
         if mixed:
             # increments: u (float), r - u (float), nu in; delta out

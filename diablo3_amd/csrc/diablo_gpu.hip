@@ -427,8 +427,8 @@ int ensure_fft_scratch(dgpu_handle* h) {
 // per-kernel timing
 // --------------------------------------------------------------------------------
 constexpr int NKERN = 13;
-const char* const kKernelNames[NKERN] = {"k_inv_z",   "k_les_products", "k_fwdz_nl", "k_cn",      "k_project",
-                                         "k_bc_post", "les_grad",       "",          "k_cn_phys", "les_cn_fft",
+const char* const kKernelNames[NKERN] = {"k_inv_z",   "k_les_products", "k_fwdz_nl", "k_assemble", "k_project",
+                                         "k_bc_post", "les_grad",       "unused",    "k_cn_phys",  "les_cn_fft",
                                          "k_closure", "k_xmarch",       "k_column"};
 
 hipEvent_t pool_event(dgpu_handle* h) {
@@ -1202,7 +1202,7 @@ int substep(dgpu_handle* h, int rk, double delta_t, double time, int time_step, 
   // courant reads the new velocity before the projection (for/solver.f90:1241-1244):
   // the column pass stops after the solves then, and the projection follows it
   const bool courant_now = h->variable_dt && rk == 3 && time_step % h->update_dt == 0;
-  if ((rc = tbeg(h, courant_now ? 3 : 12))) return rc;
+  if ((rc = tbeg(h, 12))) return rc;
   rc = launch_column(ca, cs, h->nth, mixed, courant_now ? 0 : 1, h->st);
   if (rc || (rc = tend(h))) return rc;
   if (!courant_now) return 0;

@@ -181,15 +181,16 @@ int dgpu_last_step_ms(dgpu_handle *h, double *ms);
 /* Per-kernel device timing, for measurement only (no counterpart in the
  * reference).  While enabled, every launch of the step's kernels is bracketed by
  * HIP events on the handle's stream.  Kernel ids: 0 = z inverse transform of the
- * state, 1 = the LES x pass (model, products and their forward x
- * transforms), 2 = z forward transform of the products, 3 = Fourier assembly (LES; with the Crank-Nicolson solves where courant follows
- * them in a DNS substep), 4 = projection + pressure update (LES, and after courant);
+ * state, 1 = the LES x pass (model, products and their forward x transforms),
+ * 2 = z forward transform of the products, 3 = Fourier assembly (LES), 4 = projection
+ * + pressure update (LES, and DNS substeps in which courant runs before it);
  * LES substeps add 5 = BC posts, 6 = gradient fields, 7 = not used,
  * 8 = physical-column CN solves, 9 = right-hand-side and solution transforms,
  * 10 = the learned closure's coefficients (les_model_type 6, dgpu_closure.h),
  * 11 = the DNS x pass (x inverse transforms, products and x forward transforms
  * in one kernel marching in y), 12 = the DNS column pass (Fourier assembly,
- * Crank-Nicolson solves, projection and pressure update in one kernel).
+ * Crank-Nicolson solves and, but for the substeps in which courant follows the
+ * solves, projection and pressure update in one kernel).
  * dgpu_timing_read returns the device time and launch count accumulated since the
  * last enable, and the name.  Enabling resets the dgpu_step sampling to every call. */
 int dgpu_timing_enable(dgpu_handle *h, int32_t enable);
