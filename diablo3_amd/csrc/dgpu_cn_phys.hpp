@@ -175,20 +175,16 @@ __global__ __launch_bounds__(CN_PHYS_NT) void k_cn_phys(PhysCnArgs<TU, TV> a) {
     __builtin_amdgcn_sched_barrier(0);  // one row at a time: interleaved rows cost registers
   }
   // the chunk's last row, and its first row as x_0 = f - fa x_L - fe x_R
-  constexpr int LS = RPT >= 2 ? RPT - 2 : 0;
-  const bool some = full || RPT >= 2;  // a chunk of RPT = 1 may be empty
-  double sa = some ? (full ? A[RPT - 1] : A[LS]) : 0.0, sq = some ? (full ? Q[RPT - 1] : Q[LS]) : 0.0;
-  double sg = some ? (full ? G[RPT - 1] : G[LS]) : 0.0;
-  double fa = 0.0, fe = 0.0, f = 0.0;
-  if constexpr (RPT >= 2) {
-    fa = full ? A[LS] : 0.0; fe = full ? Q[LS] : 0.0; f = full ? G[LS] : 0.0;
+  static_assert(RPT >= 2, "every chunk has a row");
+  constexpr int LS = RPT - 2;  // the last row of a chunk of RPT - 1
+  const double sa = full ? A[RPT - 1] : A[LS], sq = full ? Q[RPT - 1] : Q[LS], sg = full ? G[RPT - 1] : G[LS];
+  double fa = full ? A[LS] : 0.0, fe = full ? Q[LS] : 0.0, f = full ? G[LS] : 0.0;
 #pragma unroll
-    for (int m = RPT - 3; m >= 0; --m) {
-      const bool first = m == RPT - 3 && !full;  // the row above a short chunk's last
-      fa = first ? A[m] : A[m] - Q[m] * fa;
-      f = first ? G[m] : G[m] - Q[m] * f;
-      fe = first ? Q[m] : -(Q[m] * fe);
-    }
+  for (int m = RPT - 3; m >= 0; --m) {
+    const bool first = m == RPT - 3 && !full;  // the row above a short chunk's last
+    fa = first ? A[m] : A[m] - Q[m] * fa;
+    f = first ? G[m] : G[m] - Q[m] * f;
+    fe = first ? Q[m] : -(Q[m] * fe);
   }
   double *cur = sx, *nxt = sx + 3 * NT;
   auto put = [&](double* b, double x, double y, double z) { b[tid] = x; b[NT + tid] = y; b[2 * NT + tid] = z; };

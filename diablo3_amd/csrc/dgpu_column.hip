@@ -35,12 +35,13 @@ template int launch_column_t<double>(const ColArgs&, const ColShape&, int, int, 
 // 232, 382).  32 chunks (256 threads, two blocks per CU) up to 5 rows each (5 rows:
 // 179 us; 64 chunks of 3: 249), then 64 chunks up to the 320 rows whose tables fit
 // LDS (512x257x512 DNS mixed, 64 chunks of 5: 1449 us; 4 columns 1648).  Taller
-// columns, and fields of 4 GiB and more (32-bit offsets), take narrower blocks
-// with the tables in global memory.
+// columns take narrower blocks with the tables in global memory, and 64-bit offsets (up
+// to 320 rows the widest field is below 4 GiB).
+static_assert(344ll * 683 * COLUMN_ROWS * 16 < (1ll << 32), "kxp kzr of 1024 x 1024 points");
 bool column_shape(const Geo& g, ColShape* s) {
   const int n2 = g.ny2;
   int tc = 8, P = n2 <= 160 ? 32 : 64;
-  const bool big = n2 > COLUMN_ROWS || g.pc * n2 >= (1ll << 28);
+  const bool big = n2 > COLUMN_ROWS;
   if (big) {
     tc = n2 <= 640 ? 4 : 2;
     P = n2 <= 640 ? 128 : 256;

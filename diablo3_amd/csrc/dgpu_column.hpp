@@ -37,6 +37,11 @@ namespace dgpu {
 constexpr int COLUMN_NT = 512;    // threads per block at most: 256 registers per thread
 constexpr int COLUMN_ROWS = 320;  // rows whose tables fit LDS beside the exchange (8 columns, 5 rows a chunk)
 
+// The tallest column a DNS step takes: 80 KiB of right-hand sides (16 bytes a row and
+// field), a limit of the interface.  No kernel holds them any more; the projection and
+// the LES step take every row count of a handle.
+__host__ __device__ constexpr int column_max_rows(int nth) { return 80 * 1024 / (16 * (3 + nth)); }
+
 // Columns per block, chunks per column (a power of two), rows per chunk: a chunk
 // holds rpt or rpt - 1 rows.
 struct ColShape {

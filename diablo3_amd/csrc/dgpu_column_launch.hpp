@@ -32,16 +32,23 @@ int run_column(const ColArgs& a, int P, int project, hipStream_t st) {
   return e == hipSuccess ? 0 : set_error(10, std::string("k_column: ") + hipGetErrorString(e));
 }
 
+// whether a column of the rows that k_column takes can have RPT rows a chunk (two
+// columns a block run with 256 chunks)
+template <int NTH, int TC, int RPT>
+constexpr bool column_reaches = TC > 2 || (RPT - 1) * 256 < column_max_rows(NTH);
+
 template <typename T>
 int launch_column_t(const ColArgs& a, const ColShape& s, int nth, int project, hipStream_t st) {
+#define DG_N(NTH_, TC_, RPT_, BIG_)                                                     \
+  if constexpr (column_reaches<NTH_, TC_, RPT_>)                                        \
+    if (nth == NTH_) return run_column<T, NTH_, TC_, RPT_, BIG_>(a, s.P, project, st);
 #define DG_X(TC_, RPT_, BIG_)                                                           \
   if (s.tc == TC_ && s.rpt == RPT_ && s.big == BIG_) {                                  \
-    if (nth == 0) return run_column<T, 0, TC_, RPT_, BIG_>(a, s.P, project, st);        \
-    if (nth == 1) return run_column<T, 1, TC_, RPT_, BIG_>(a, s.P, project, st);        \
-    if (nth == 2) return run_column<T, 2, TC_, RPT_, BIG_>(a, s.P, project, st);        \
+    DG_N(0, TC_, RPT_, BIG_) DG_N(1, TC_, RPT_, BIG_) DG_N(2, TC_, RPT_, BIG_)          \
   }
   DG_COLUMN_SHAPES(DG_X)
 #undef DG_X
+#undef DG_N
   return set_error(2, "ny too large for the column kernels");
 }
 #endif

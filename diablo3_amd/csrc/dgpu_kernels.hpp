@@ -313,8 +313,7 @@ struct XProdArgs {
   Geo g;
   int jlo;
   int jstart, jend, jstart_th[MAXTH], jend_th[MAXTH];
-  const double* __restrict__ dy;
-  const double* __restrict__ dyf;
+  const double* __restrict__ dyf;   // k_xmarch, as rowc and hin (the LES pass has AmdArgs)
   const double* __restrict__ rowc;  // [ny2][RC_COUNT] grid quotients
   const double* __restrict__ kx;
   const void* hin[MAXF];   // x-spectra of u1, u2, u3, th_n (all planes)
@@ -684,19 +683,17 @@ struct ColArgs {
   Geo g;
   int rk;
   int cr_minus_u;   // k_assemble: write the right-hand side minus the state (increment solves)
-  int jstart, jend, jstart_th[MAXTH], jend_th[MAXTH];
-  int front, f_type;
-  double nu, beta, nu_v_scale, ro_inv, delta, grav_x, grav_y, grav_z, ly, px0, omega0, amp_omega0, time;
-  double pr[MAXTH], dthdx[MAXTH], dthdz[MAXTH];
-  double temp1, temp3, temp4, temp5;
+  int jstart, f_type;
+  double nu, beta, grav_x, grav_y, grav_z, px0, omega0, amp_omega0, time;
+  double dthdx[MAXTH], dthdz[MAXTH];
+  double temp3, temp4, temp5;
   // host-precomputed scalars: Ro_inv/delta; the scalars' sums of dthdx delta/Ro_inv
   // and -dthdz delta/Ro_inv (0 without the thermal wind); per scalar nu/Pr,
   // temp1 nu_v_scale/Pr; temp1 nu_v_scale
   double cori, twu_x, twu_z, nupr[MAXTH], t1pr[MAXTH], t1v;
   double twon;   // 1 with the front's thermal-wind terms, else 0
   const double* __restrict__ rowc;  // [ny2][RC_COUNT]
-  const double *__restrict__ dy, *__restrict__ dyf, *__restrict__ gy, *__restrict__ gyf;
-  const double *__restrict__ kx, *__restrict__ kz;
+  const double *__restrict__ gyf, *__restrict__ kx, *__restrict__ kz;
   SolveRows rows[MAXF];
   unsigned long long bcmask;  // bit MAXF s + e: row s of SolveRows::kind is a BC row of field e
   // Thomas factorisation of the CN systems, [field][3][ny2]: mu_j (forward

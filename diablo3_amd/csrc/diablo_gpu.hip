@@ -324,10 +324,6 @@ int thomas_chunk_coefficients(const std::vector<double>& a, const std::vector<do
   return 0;
 }
 
-// The step takes columns of at most 80 KiB of right-hand sides (16 (3 + N_th)
-// bytes a row); taller ones are refused.
-bool column_rows_ok(const dgpu_handle* h) { return (size_t)h->g.ny2 * 16 * (3 + h->nth) <= 80 * 1024; }
-
 int ensure_factors(dgpu_handle* h, double delta_t) {
   if (h->fac_dt == delta_t) return 0;
   const int n2 = h->c.ny + 2, nf = 3 + h->nth;
@@ -335,7 +331,7 @@ int ensure_factors(dgpu_handle* h, double delta_t) {
   std::vector<double> buf((size_t)3 * MAXF * per_field, 0.0), a, b, cc;
   const double hb[3] = {delta_t * (8.0 / 15.0), delta_t * (2.0 / 15.0), delta_t * (5.0 / 15.0)};
   ColShape cs{};
-  if (!column_rows_ok(h) || !column_shape(h->g, &cs)) return fail(2, "ny too large for the column kernels");
+  if (n2 > column_max_rows(h->nth) || !column_shape(h->g, &cs)) return fail(2, "ny too large for the column kernels");
   for (int r = 0; r < 3; ++r) {
     const double temp1 = 0.5 * h->c.nu * hb[r];
     for (int F = 0; F < nf; ++F) {
@@ -748,14 +744,11 @@ int download_field(dgpu_handle* h, const cd* dev, double* fort) {
 void fill_col_args(dgpu_handle* h, ColArgs& ca, double time) {
   const dgpu_config& c = h->c;
   ca.g = h->g;
-  ca.jstart = c.jstart; ca.jend = c.jend;
-  for (int n = 0; n < MAXTH; ++n) {
-    ca.jstart_th[n] = c.jstart_th[n]; ca.jend_th[n] = c.jend_th[n];
-    ca.pr[n] = c.pr[n]; ca.dthdx[n] = c.dthdx[n]; ca.dthdz[n] = c.dthdz[n];
-  }
-  ca.front = c.flavor_front; ca.f_type = c.f_type;
-  ca.nu = c.nu; ca.beta = c.beta; ca.nu_v_scale = c.nu_v_scale; ca.ro_inv = c.ro_inv; ca.delta = c.delta;
-  ca.grav_x = c.grav_x; ca.grav_y = c.grav_y; ca.grav_z = c.grav_z; ca.ly = c.ly;
+  ca.jstart = c.jstart;
+  for (int n = 0; n < MAXTH; ++n) { ca.dthdx[n] = c.dthdx[n]; ca.dthdz[n] = c.dthdz[n]; }
+  ca.f_type = c.f_type;
+  ca.nu = c.nu; ca.beta = c.beta;
+  ca.grav_x = c.grav_x; ca.grav_y = c.grav_y; ca.grav_z = c.grav_z;
   ca.px0 = c.px0; ca.omega0 = c.omega0; ca.amp_omega0 = c.amp_omega0; ca.time = time;
   ca.temp4 = 1.0;
   ca.cori = c.ro_inv / c.delta;
@@ -770,7 +763,7 @@ void fill_col_args(dgpu_handle* h, ColArgs& ca, double time) {
     ca.nupr[n] = n < h->nth ? c.nu / c.pr[n] : 0.0;
   }
   ca.rowc = h->d_rowc;
-  ca.dy = h->d_dy; ca.dyf = h->d_dyf; ca.gy = h->d_gy; ca.gyf = h->d_gyf; ca.kx = h->d_kx; ca.kz = h->d_kz;
+  ca.gyf = h->d_gyf; ca.kx = h->d_kx; ca.kz = h->d_kz;
   solve_rows(h, time, ca.rows);
   ca.bcmask = 0;
   for (int f = 0; f < 3 + h->nth; ++f)
@@ -1008,8 +1001,7 @@ int substep_les(dgpu_handle* h, int rk, double delta_t, double time, int time_st
   XProdArgs xa{};
   xa.g = g; xa.jlo = jlo; xa.jstart = c.jstart; xa.jend = c.jend;
   for (int n = 0; n < MAXTH; ++n) { xa.jstart_th[n] = c.jstart_th[n]; xa.jend_th[n] = c.jend_th[n]; }
-  xa.dy = h->d_dy; xa.dyf = h->d_dyf; xa.kx = h->d_kx; xa.rowc = h->d_rowc;
-  for (int f = 0; f < nf; ++f) xa.hin[f] = h->Hin[f];
+  xa.kx = h->d_kx;
   for (int o = 0; o < 6 + 2 * NTH; ++o) xa.hout[o] = h->Hout[o];
   if ((rc = tbeg(h, 1))) return rc;
   if (c.les_model_type == 1) rc = launch_les_products<T, NTH, 1>(h, xa, aa, nj);
@@ -1032,7 +1024,7 @@ int substep_les(dgpu_handle* h, int rk, double delta_t, double time, int time_st
   ColArgs ca{};
   fill_col_args(h, ca, time);
   ca.rk = rk;
-  ca.temp1 = temp1; ca.temp3 = temp3; ca.temp4 = temp4; ca.temp5 = temp5;
+  ca.temp3 = temp3; ca.temp4 = temp4; ca.temp5 = temp5;
   ca.t1v = temp1 * c.nu_v_scale;
   for (int n = 0; n < NTH; ++n) ca.t1pr[n] = temp1 / c.pr[n] * c.nu_v_scale;
   // the mixed handle solves for the increment of the state in float transforms,
@@ -1170,7 +1162,7 @@ int substep(dgpu_handle* h, int rk, double delta_t, double time, int time_step, 
   XProdArgs xa{};
   xa.g = g; xa.jlo = jlo; xa.jstart = c.jstart; xa.jend = c.jend;
   for (int n = 0; n < MAXTH; ++n) { xa.jstart_th[n] = c.jstart_th[n]; xa.jend_th[n] = c.jend_th[n]; }
-  xa.dy = h->d_dy; xa.dyf = h->d_dyf; xa.kx = h->d_kx; xa.rowc = h->d_rowc;
+  xa.dyf = h->d_dyf; xa.kx = h->d_kx; xa.rowc = h->d_rowc;
   for (int f = 0; f < nf; ++f) xa.hin[f] = h->Hin[f];
   for (int o = 0; o < 6 + 2 * h->nth; ++o) xa.hout[o] = h->Hout[o];
   if ((rc = tbeg(h, 11))) return rc;
@@ -1193,7 +1185,7 @@ int substep(dgpu_handle* h, int rk, double delta_t, double time, int time_step, 
   ColArgs ca{};
   fill_col_args(h, ca, time);
   ca.rk = rk;
-  ca.temp1 = temp1; ca.temp3 = temp3; ca.temp4 = temp4; ca.temp5 = temp5;
+  ca.temp3 = temp3; ca.temp4 = temp4; ca.temp5 = temp5;
   ca.t1v = temp1 * c.nu_v_scale;
   for (int n = 0; n < h->nth; ++n) ca.t1pr[n] = temp1 / c.pr[n] * c.nu_v_scale;
   ca.thc = h->d_fac + (size_t)r * MAXF * 3 * g.ny2;
