@@ -546,22 +546,31 @@ __global__ __launch_bounds__(COLUMN_NT) void k_project(ColArgs a, int update_p) 
   cd v1[RPT], v2[RPT], v3[RPT], d[RPT];
   if (a.prhs) {
     // poisson_p_chan (for/solver.f90:1382-1560): vec = -(source + the scalars' y
-    // gradient, except in the (0, 0) mode)
+    // gradient, except in the (0, 0) mode).  Rows past the chunk are read in bounds and
+    // dropped, as below: loads under a row's own condition wait for one another
+    // (poisson_p with its transforms, us: 64x65x64 58.8 -> 57.7, 256x129x256 665 -> 656,
+    // 64x385x64 158.5 -> 152.1; the kernel of one row a thread before it 57.2, 657, 154)
+    double yf[RPT + 2];
+    auto row = [&](int m) { const int j = j0 - 1 + m; return j < 0 ? 0 : (j >= n2 ? n2 - 1 : j); };
+#pragma unroll
+    for (int m = 0; m < RPT; ++m) d[m] = a.prhs[(long long)row(m + 1) * pc + c];
+#pragma unroll
+    for (int m = 0; m < RPT + 2; ++m) yf[m] = a.gyf[row(m)];
+    for (int n = 0; n < a.pnth; ++n) {
+      cd t[RPT + 2];
+#pragma unroll
+      for (int m = 0; m < RPT + 2; ++m) t[m] = a.u[3 + n][(long long)row(m) * pc + c];
+#pragma unroll
+      for (int m = 0; m < RPT; ++m) {
+        const cd dt = t[m + 2] - t[m];
+        const double den = yf[m + 2] - yf[m];
+        d[m] = pick(c != 0, d[m] + cd{dt.x / den, dt.y / den}, d[m]);
+      }
+    }
 #pragma unroll
     for (int m = 0; m < RPT; ++m) {
       const int j = j0 + m;
-      d[m] = cd{0.0, 0.0};
-      if ((m + 1 < RPT || full) && j > 1 && j < ny && active) {
-        const long long o = (long long)j * pc + c;
-        cd sv = a.prhs[o];
-        if (c != 0)
-          for (int n = 0; n < a.pnth; ++n) {
-            const cd dt = a.u[3 + n][o + pc] - a.u[3 + n][o - pc];
-            const double den = a.gyf[j + 1] - a.gyf[j - 1];
-            sv = sv + cd{dt.x / den, dt.y / den};
-          }
-        d[m] = -1.0 * sv;
-      }
+      d[m] = pick((m + 1 < RPT || full) && j > 1 && j < ny && active, -1.0 * d[m], cd{0.0, 0.0});
     }
     __syncthreads();  // the row coefficients
   } else {
