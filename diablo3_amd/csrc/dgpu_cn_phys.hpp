@@ -28,9 +28,12 @@ namespace dgpu {
 // 72 bytes a point and field against 32, in float 40 against 16.)  With the rows
 // of a column nx values apart (the [z][j][x] layout) a block stays within one or
 // two pages; plane after plane (a 2 MB stride at 512x512) the same kernel took
-// 2546 us.  Measured, one thread per column -> this: 512x257x512 FP64 3852 -> 1855 us
-// (4.7 TB/s, the rate of a large copy), mixed 2038 -> 1210 (3.6 TB/s; the FP64
-// arithmetic of a row takes as long as its 16 bytes); 128x129x128 FP64 252 -> 60.
+// 2546 us.  Measured, one thread per column -> this: 512x257x512 FP64 3852 -> 1855 us,
+// mixed 2038 -> 1207; 128x129x128 FP64 252 -> 60; 1024x385x1024 mixed 10.5-11.2 ->
+// 11.9 ms.  FP64 moves 7.6 GB (nu_t is found in L2), 4.1 TB/s of the 5.7 of a large
+// one-read-one-write pass, with waves waiting 41% of their cycles.  Mixed moves 6.5 GB
+// where 4.3 would do, and that traffic (5.4 TB/s) bounds it: a block's 16 float columns
+// are half a 128-byte line, and the block with the other half runs on another XCD.
 //
 // INC (the mixed-precision path): u is the state at the substep's start in
 // float and r holds r - u (float).  The solve is then for the increment

@@ -14,19 +14,25 @@
 //
 // A block owns TC columns; thread (p, cc) owns the rows of chunk p of column cc,
 // RPT of them at most, and keeps them in registers from the assembly to the
-// corrected velocity: every state field is read once and written once (641 MB a
-// substep at 256x129x256 FP64, against 889 MB of an assembly + solve kernel that
-// kept its right-hand sides in LDS and a projection kernel that read the velocity
-// back).  What crosses chunks is small and goes through shuffles (the chunks of
+// corrected velocity: with every state field read once and written once 632 MB a
+// substep at 256x129x256 FP64.  Counted, it is 793 MB (516 in, 277 out): a chunk reads
+// the rows next to it again, and a short chunk (29 of 32 there) the row it does not
+// own.  (942 MB counted for an assembly + solve kernel that kept its right-hand sides
+// in LDS and a projection kernel that read the velocity back.)  What crosses chunks is
+// small and goes through shuffles (the chunks of
 // one wave) and LDS (the waves of a block): the carries of the two Thomas sweeps,
 // and the Poisson system of the chunks' last rows.
 //
 // Measured (MI355X, per substep, those two kernels -> k_column): 256x129x256 FP64
-// 268 -> 179 us (3.6 TB/s), mixed 269 -> 169; 64x65x64 FP64 23.5 -> 20.7;
-// 128x97x64 mixed, two scalars 55 -> 37.  k_project alone (LES), 512x257x512: 709 ->
-// 528 us.  What bounds k_column is the length of one block's chain (rows one
-// after another, then the scans and log2 P exchange steps) at the two blocks per
-// CU that 256 registers a thread allow.
+// 268 -> 179 us, mixed 269 -> 169; 64x65x64 FP64 23.5 -> 18.4; 128x97x64 mixed, two
+// scalars 55 -> 37.  k_project alone (LES), 512x257x512: 709 -> 520 us.  What bounds
+// k_column is that traffic (4.4 TB/s; a large one-read-one-write pass reaches 5.7) and
+// the length of one block's chain (rows one after another, then the scans and log2 P
+// exchange steps): waves wait 44% of their cycles, at 1.5 waves per SIMD, which 256
+// registers a thread allow (5 rows and one scalar: all 256, and 12 bytes of scratch).
+// On the smallest grids the chain is all of it: with 11 blocks (16 points in x and z) it
+// takes up to 1 us longer than the two kernels, whose blocks were narrower (a step of
+// 16x65x16 103 -> 105 us; 32x65x32 122 -> 119).
 #pragma once
 #include "dgpu_kernels.hpp"
 

@@ -641,8 +641,9 @@ __device__ __forceinline__ void les_store(const cx<T>* __restrict__ s, const Geo
 // once; the 7 + 2 N_th SGS fields a separate model kernel wrote and the product
 // kernel read back never reach memory.  Planes follow one another on an XCD
 // (blocks b, b + 8, ...), so that the rows j - 1 .. j + 2 a block reads are in its L2.
-// Memory traffic bounds it in float; in FP64 the model's arithmetic and the
-// transforms cost as much, and the blocks of a CU overlap them.
+// In float the vector instructions bound it (845 per 64 points, 90% of the issue slots;
+// 5.3 GB, the bytes of its fields, at 2.9 TB/s); in FP64 the two waves per SIMD that
+// 255 registers leave (54% of the issue slots, 10.5 GB at 3.3 TB/s).
 //
 // SPLIT: the lines of u1's and u3's equations are transformed first, those of u2's
 // and the scalars' held in registers meanwhile, so that the tile is half the size

@@ -4,7 +4,7 @@ coefficients the step uses, from the type-5 quantities the oracle captures
 (oracle_les_capture) and the network of oracle/mlp.py.
 
 TEST INFRASTRUCTURE ONLY (imported by tests/): the checker of the device's
-k_closure and k_amd<..., 6>.  The learned closure has no counterpart in the
+k_closure and k_les_products (model 6).  The learned closure has no counterpart in the
 reference; it replaces the AMD coefficient of les_chan / les_chan_th type 5
 (for/les.f90:571-797, 1201-1348) by the network's prediction.
 
