@@ -30,10 +30,11 @@ extern template int launch_column_t<float>(const ColArgs&, const ColShape&, int,
 template int launch_column_t<double>(const ColArgs&, const ColShape&, int, int, hipStream_t);
 
 // 8 columns a block: a wave's load then takes whole 128-byte lines, and narrower
-// blocks were slower even on the grids that leave CUs idle (64x65x64, 129 blocks:
-// k_column 20.7 us; 4 columns, 258 blocks, 23.6; 2 columns 27.4.  256x129x256: 179,
-// 232, 382).  32 chunks (256 threads, two blocks per CU) up to 5 rows each (5 rows:
-// 179 us; 64 chunks of 3: 249), then 64 chunks up to the 320 rows whose tables fit
+// blocks were slower even on the grids that leave CUs idle (one comparison, k_column
+// alone: 64x65x64, 129 blocks, 20.7 us; 4 columns, 258 blocks, 23.6; 2 columns 27.4.
+// 256x129x256: 179, 232, 382).  32 chunks (256 threads, two blocks per CU) up to 5 rows each (5 rows:
+// 179 us; 64 chunks of 3: 249; a step of 32x65x32 119 us, with 64 chunks 130, with 16 125;
+// of 16x33x16, two scalars, 104, 114, 104), then 64 chunks up to the 320 rows whose tables fit
 // LDS (512x257x512 DNS mixed, 64 chunks of 5: 1449 us; 4 columns 1648).  Taller
 // columns take narrower blocks with the tables in global memory, and 64-bit offsets (up
 // to 320 rows the widest field is below 4 GiB).
